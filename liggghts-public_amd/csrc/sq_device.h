@@ -1,11 +1,14 @@
-// Superquadric contact-point solve on the device, FP64, one thread per pair.
-// Same arithmetic and control flow as the reference's
+// Superquadric shape functions, the pieces of the contact-point solve, and
+// contact detection around the point, on the device in FP64, one thread per
+// pair; the solve itself (calc_contact_point and its homotopy) runs on eight
+// lanes per pair (sq_group.h). Same arithmetic and control flow as the
+// reference's
 //   Superquadric::shape_function_props_local/_global (superquadric.cpp:237-326),
 //   calc_F (math_extra_liggghts_superquadric.cpp:619-658),
 //   determinant_4x4 / inverseMatrix4x4 (:715-775),
 //   GMRES<4,4> (math_extra_liggghts_nonspherical.h:225-314),
-//   calc_contact_point (math_extra_liggghts_superquadric.cpp:778-1022) and the
-//   homotopy of calc_contact_point_if_no_previous_point_avaialable (:1390-1430),
+//   surface_line_intersection (superquadric.cpp:712-816) and the OBB test
+//   (math_extra_liggghts_superquadric.cpp:72-203),
 // written for registers: fixed-size arrays, no heap, no recursion.
 #pragma once
 
@@ -372,177 +375,6 @@ __device__ __forceinline__ void cp4(double *d, const double *s) {
   d[3] = s[3];
 }
 
-// calc_contact_point; returns Newton iterations, sets fail
-__device__ __forceinline__ int contact_point(Sq &A, Sq &B, double ratio, const double *init1, double *result,
-                                          double &fi, double &fj, int &fail, int max_iter) {
-  const double tol1 = 1e-10, tol2 = 1e-12;
-  fail = 0;
-  double mu, mu_sq, F[4], F1[4], F2[4], point[3];
-  double mu1, mu2, gA1[3], gB1[3], gA2[3], gB2[3];
-  double fi1, fj1, fi2, fj2, merit01, merit02, merit0;
-  const double res01 = calc_F_free(A, B, fi1, fj1, gA1, gB1, init1, mu1, F1, merit01);
-  if (merit01 < tol1) {
-    cp3(result, init1);
-    cp3(A.gradient, gA1);
-    cp3(B.gradient, gB1);
-    fi = fi1;
-    fj = fj1;
-    return 0;
-  }
-  double init2[3];
-  for (int k = 0; k < 3; k++) init2[k] = ratio * B.center[k] + (1.0 - ratio) * A.center[k];
-  const double res02 = calc_F_free(A, B, fi2, fj2, gA2, gB2, init2, mu2, F2, merit02);
-  double res0;
-  if (res01 < res02) {
-    res0 = res01;
-    cp3(A.gradient, gA1);
-    cp3(B.gradient, gB1);
-    cp3(point, init1);
-    cp4(F, F1);
-    fi = fi1;
-    fj = fj1;
-    mu = mu1;
-    merit0 = merit01;
-  } else {
-    res0 = res02;
-    cp3(A.gradient, gA2);
-    cp3(B.gradient, gB2);
-    cp3(point, init2);
-    cp4(F, F2);
-    fi = fi2;
-    fj = fj2;
-    mu = mu2;
-    merit0 = merit02;
-  }
-  if (merit0 < tol1) {
-    cp3(result, point);
-    return 0;
-  }
-  double merit1 = merit0, merit2 = merit0, res1 = res0, res2 = res1;
-  const double size_i = fmin(fmin(A.shape[0], A.shape[1]), A.shape[2]);
-  const double size_j = fmin(fmin(B.shape[0], B.shape[1]), B.shape[2]);
-  const double size = size_i < size_j ? size_i : size_j;
-  double J4[16], J4inv[16], delta[4] = {0, 0, 0, 0}, delta_0[4], pointa[3], pointb[3];
-  int iter;
-  for (iter = 0; iter < max_iter; iter++) {
-    merit2 = merit1;
-    res2 = res1;
-    {
-      double fd, gd[3];
-      props_global<true>(A, point, fd, gd, A.hessian);
-      props_global<true>(B, point, fd, gd, B.hessian);
-    }
-    mu_sq = mu * mu;
-    for (int i = 0; i < 3; i++) {
-      for (int j = 0; j < 3; j++) J4[4 * i + j] = A.hessian[i * 3 + j] + mu_sq * B.hessian[i * 3 + j];
-      J4[3 + 4 * i] = 2.0 * mu * B.gradient[i];
-      J4[i + 4 * 3] = A.gradient[i] - B.gradient[i];
-    }
-    J4[15] = 0.0;
-    const double det = det4(J4);
-    if (fabs(det) > 1.0) {
-      inv4(J4, J4inv);
-      matvec4(J4inv, F, delta);
-    } else {
-      cp4(delta_0, delta);
-      gmres44(J4, F, delta_0, delta);
-    }
-    int nan_found = 0;
-    for (int i = 0; i < 4; i++)
-      if (isnan(delta[i])) {
-        nan_found = 1;
-        fail = 1;
-        break;
-      }
-    int converged = 0;
-    const double deltax = fmax(fmax(fabs(delta[0]), fabs(delta[1])), fabs(delta[2]));
-    if (deltax == 0.0) {
-      cp3(result, point);
-      converged = 1;
-    } else {
-      if (nan_found) break;
-      double point_[3], fi_, fj_, merit2_;
-      for (int k = 0; k < 3; k++) point_[k] = point[k] - delta[k];
-      const double mu_ = mu - delta[3];
-      const double res2_ = calc_F_mu(A, B, fi_, fj_, A.gradient, B.gradient, point_, mu_, F, merit2_);
-      if (res2_ < res1 || merit2_ < tol1 || deltax < tol2 * size) {
-        merit2 = merit2_;
-        res2 = res2_;
-        mu = mu_;
-        fi = fi_;
-        fj = fj_;
-        cp3(point, point_);
-        if (merit2 < tol1 || deltax < tol2 * size) converged = 1;
-      } else {
-        double a = 0.0, b = 1.0, eps = fabs(b - a);
-        double res2a = 0, res2b = 0, merit2a = 0, merit2b = 0;
-        while (eps > 1e-8) {
-          const double alpha1 = b - (b - a) * kPhiInv;
-          const double alpha2 = a + (b - a) * kPhiInv;
-          for (int k = 0; k < 3; k++) pointa[k] = point[k] + (-alpha1) * delta[k];
-          mu1 = mu - alpha1 * delta[3];
-          res2a = calc_F_mu(A, B, fi1, fj1, gA1, gB1, pointa, mu1, F1, merit2a);
-          for (int k = 0; k < 3; k++) pointb[k] = point[k] + (-alpha2) * delta[k];
-          mu2 = mu - alpha2 * delta[3];
-          res2b = calc_F_mu(A, B, fi2, fj2, gA2, gB2, pointb, mu2, F2, merit2b);
-          if ((res2a < res2b ? res2a : res2b) < res1) {
-            if (res2a < res2b) {
-              res2 = res2a;
-              cp4(F, F1);
-              mu = mu1;
-              cp3(A.gradient, gA1);
-              cp3(B.gradient, gB1);
-              cp3(point, pointa);
-              fi = fi1;
-              fj = fj1;
-              merit2 = merit2a;
-            } else {
-              res2 = res2b;
-              cp4(F, F2);
-              mu = mu2;
-              cp3(A.gradient, gA2);
-              cp3(B.gradient, gB2);
-              cp3(point, pointb);
-              fi = fi2;
-              fj = fj2;
-              merit2 = merit2b;
-            }
-            if (merit2 < tol1) converged = 1;
-            eps = 0.0;
-          } else {
-            if (res2a > res2b)
-              a = alpha1;
-            else
-              b = alpha2;
-            eps = fabs(b - a);
-          }
-        }
-        if (eps != 0.0) {
-          cp4(F, F2);
-          mu = mu2;
-          cp3(A.gradient, gA2);
-          cp3(B.gradient, gB2);
-          cp3(point, pointb);
-          fi = fi2;
-          fj = fj2;
-          res2 = res2b;
-          merit2 = merit2b;
-          if (merit2 < tol1) converged = 1;
-        }
-      }
-      if (fabs(res1 - res2) / fmax(res1, res2) < 1e-3) converged = 1;
-    }
-    merit1 = merit2;
-    res1 = res2;
-    if (iter >= max_iter - 1) fail = 1;
-    if (converged || fail) {
-      cp3(result, point);
-      break;
-    }
-  }
-  return iter + 1;
-}
-
 // Extra full Newton steps on the converged system (F = 0, f_A = f_B) from
 // point cp, each kept only if it lowers the residual; stops after `steps`,
 // at a residual below 1e-30 or when a step does not help. Not part of the
@@ -587,40 +419,6 @@ __device__ __forceinline__ int polish(Sq &A, Sq &B, double *cp, double &fi, doub
     done++;
   }
   return done;
-}
-
-// the homotopy from volume-equivalent spheres (N+1 solves)
-__device__ __forceinline__ int contact_point_fresh(Sq &A, Sq &B, double *cp, double &fi, double &fj, int &fail,
-                                                int max_iter) {
-  const double ai = A.shape[0], bi = A.shape[1], ci = A.shape[2];
-  const double aj = B.shape[0], bj = B.shape[1], cj = B.shape[2];
-  const double ri = cbrt(ai * bi * ci), rj = cbrt(aj * bj * cj);
-  const double ratio = ri / (ri + rj);
-  const double ni0 = A.blk[0], ni1 = A.blk[1], nj0 = B.blk[0], nj1 = B.blk[1];
-  const double nmax = fmax(fmax(fmax(ni0, ni1), nj0), nj1);
-  const int N1 = (int)((nmax - 2.0) / 1.0 + 1);
-  const int N = N1 > 10 ? N1 : 10;
-  const double Ninv = 1.0 / (double)N;
-  int iters = 0, f = 0;
-  fail = 0;
-  for (int i = 0; i <= N; i++) {
-    set_blockiness(A, 2.0 + (ni0 - 2.0) * (double)i * Ninv, 2.0 + (ni1 - 2.0) * (double)i * Ninv);
-    set_blockiness(B, 2.0 + (nj0 - 2.0) * (double)i * Ninv, 2.0 + (nj1 - 2.0) * (double)i * Ninv);
-    set_shape(A, ri + (ai - ri) * (double)i * Ninv, ri + (bi - ri) * (double)i * Ninv,
-              ri + (ci - ri) * (double)i * Ninv);
-    set_shape(B, rj + (aj - rj) * (double)i * Ninv, rj + (bj - rj) * (double)i * Ninv,
-              rj + (cj - rj) * (double)i * Ninv);
-    if (i == 0)
-      for (int k = 0; k < 3; k++) cp[k] = ratio * B.center[k] + (1.0 - ratio) * A.center[k];
-    const double pre[3] = {cp[0], cp[1], cp[2]};
-    iters += contact_point(A, B, ratio, pre, cp, fi, fj, f, max_iter);
-    fail = f;
-    set_shape(A, ai, bi, ci);
-    set_shape(B, aj, bj, cj);
-    set_blockiness(A, ni0, ni1);
-    set_blockiness(B, nj0, nj1);
-  }
-  return iters;
 }
 
 // ---------------------------------------------------------------------------
@@ -765,6 +563,22 @@ __device__ __forceinline__ double line_intersection(const Sq &s, const double *s
   }
   for (int k = 0; k < 3; k++) result[k] = start[k] + alpha * dir[k];
   return alpha;
+}
+
+// The unit normal of two intersecting surfaces from their gradients at the
+// contact point cp, and where the line through cp along it leaves each
+// (extended_overlap_algorithm, math_extra_liggghts_superquadric.cpp:1489-1504):
+// the overlap is |alpha_a| + |alpha_b|
+__device__ __forceinline__ void overlap_along_normal(const Sq &A, const Sq &B, const double *cp, const double *gA,
+                                                     const double *gB, double *en, double &alpha_a,
+                                                     double &alpha_b, double *cpa, double *cpb) {
+  for (int c = 0; c < 3; c++) en[c] = gB[c] - gA[c];
+  const double nrm = sqrt(en[0] * en[0] + en[1] * en[1] + en[2] * en[2]);
+  const double inv = nrm == 0. ? 0. : 1. / nrm;
+  for (int c = 0; c < 3; c++) en[c] *= inv;
+  const double men[3] = {-en[0], -en[1], -en[2]};
+  alpha_a = line_intersection(A, cp, men, alpha_a, cpa);
+  alpha_b = line_intersection(B, cp, en, alpha_b, cpb);
 }
 
 // check_inequalities (math_extra_liggghts_superquadric.cpp:72-150): axis i

@@ -42,6 +42,7 @@ struct SolveArgs {
   int polish;                     // extra Newton refinement steps after the solve (0: none)
   double *point, *fi, *fj;
   int *iters, *fail;              // fail: bit 0 the solve's flag, bit 1 the fallback ran
+  unsigned *queue;                // next pair to be taken (the launch clears it)
 };
 
 // checkSurfaceIntersect over pose pairs; hist [n][7] = state (0 far, 1 close,
@@ -59,6 +60,7 @@ struct CheckArgs {
   double *en, *deltan, *cp_i, *cp_j;  // [n][3], [n], [n][3], [n][3]
   double *point, *fi, *fj;
   int *iters, *flags;  // flags: bit 0 the solve's flag, bit 1 the fallback ran, bit 2 no solve (OBB apart)
+  unsigned *queue;     // next pair to be taken (the launch clears it)
 };
 
 __device__ __forceinline__ unsigned short pack_bf16(float f) {

@@ -9,6 +9,7 @@
 #include <mutex>
 
 #include "sq_device.h"
+#include "sq_group.h"
 #include "sq_kernels.h"
 
 namespace sqk {
@@ -24,38 +25,55 @@ constexpr int kBlk = 256;
 
 // mode 0: fresh contacts (homotopy from spheres); mode 1: one solve from
 // init[k], and the homotopy when that one fails or stops without meeting the
-// merit tolerance (the plain start then judges and replaces it). The
-// fallback stays in the same launch: run as a separate launch over the few
-// listed pairs, the hardest homotopies would run alone on an idle GPU.
-__global__ __launch_bounds__(kBlk) void k_sq_solve(SolveArgs a) {
+// merit tolerance (the plain start then judges and replaces it).
+struct SolveSource {
+  const SolveArgs &a;
+  int64_t k;
+  __device__ bool next(sqd::QTask &t) {
+    k = sqd::q_take(a.queue, a.n);
+    if (k < 0) return false;
+    t.start = a.mode == 0 ? sqd::kStartFresh : sqd::kStartGiven;
+    for (int c = 0; c < 3; c++) {
+      t.est[c] = a.mode == 0 ? 0.0 : a.init[3 * k + c];
+      t.cp[c] = 0.0;
+    }
+    return true;
+  }
+  __device__ void pose(double *p) const {
+    const double *src = ((threadIdx.x & 8) ? a.pose_b : a.pose_a) + 12 * k;
+    for (int c = 0; c < 12; c++) p[c] = src[c];
+  }
+  __device__ void put(const sqd::QResult &r, const double *cp) const {
+    if (!sqd::q_leader()) return;
+    for (int c = 0; c < 3; c++) a.point[3 * k + c] = cp[c];
+    a.fi[k] = r.fi;
+    a.fj[k] = r.fj;
+    a.iters[k] = r.iters;
+    a.fail[k] = r.fail | (r.fallback << 1);
+  }
+};
+
+__global__ __launch_bounds__(sqd::kGroupBlock, 2) void k_sq_solve(SolveArgs a) {
+  __shared__ sqd::GroupLds lds;
+  SolveSource src{a, 0};
+  sqd::q_solve_all(src, a.max_iter, lds);
+}
+
+__global__ void k_zero_queue(unsigned *queue) { *queue = 0u; }
+
+// the optional refinement of a finished solve, one thread per pair
+__global__ __launch_bounds__(kBlk) void k_sq_polish(SolveArgs a) {
   const int64_t k = (int64_t)blockIdx.x * kBlk + threadIdx.x;
-  if (k >= a.n) return;
+  if (k >= a.n || (a.fail[k] & 1)) return;
   sqd::Sq A, B;
   sqd::init(A, a.pose_a + 12 * k);
   sqd::init(B, a.pose_b + 12 * k);
-  double cp[3], fi = 0, fj = 0;
-  int fail = 0, iters = 0, fallback = 0;
-  if (a.mode == 0) {
-    iters = sqd::contact_point_fresh(A, B, cp, fi, fj, fail, a.max_iter);
-  } else {
-    const double ri = cbrt(A.shape[0] * A.shape[1] * A.shape[2]);
-    const double rj = cbrt(B.shape[0] * B.shape[1] * B.shape[2]);
-    const double init[3] = {a.init[3 * k], a.init[3 * k + 1], a.init[3 * k + 2]};
-    iters = sqd::contact_point(A, B, ri / (ri + rj), init, cp, fi, fj, fail, a.max_iter);
-    const double merit = sqd::merit_of(A.gradient, B.gradient, fi, fj);
-    if (fail || !(merit < 1e-10)) {
-      fallback = 1;
-      iters += sqd::contact_point_fresh(A, B, cp, fi, fj, fail, a.max_iter);
-    }
-  }
-  if (a.polish > 0 && !fail) iters += sqd::polish(A, B, cp, fi, fj, a.polish);
-  a.point[3 * k] = cp[0];
-  a.point[3 * k + 1] = cp[1];
-  a.point[3 * k + 2] = cp[2];
+  double cp[3] = {a.point[3 * k], a.point[3 * k + 1], a.point[3 * k + 2]};
+  double fi = a.fi[k], fj = a.fj[k];
+  a.iters[k] += sqd::polish(A, B, cp, fi, fj, a.polish);
+  for (int c = 0; c < 3; c++) a.point[3 * k + c] = cp[c];
   a.fi[k] = fi;
   a.fj[k] = fj;
-  a.iters[k] = iters;
-  a.fail[k] = fail | (fallback << 1);
 }
 
 // SurfaceModel<SURFACE_SUPERQUADRIC>::checkSurfaceIntersect
@@ -66,8 +84,14 @@ __global__ __launch_bounds__(kBlk) void k_sq_solve(SolveArgs a) {
 // 1434-1466), and for intersecting surfaces the normal from the two gradients
 // and the overlap along it (extended_overlap_algorithm, :1489-1504). With
 // init, a pair far apart last step starts from the network's point instead of
-// the homotopy, which remains the fallback.
-__global__ __launch_bounds__(kBlk) void k_sq_check(CheckArgs a) {
+// the homotopy, which remains the fallback. Three launches: the pre-check and
+// the start point (one thread per pair), the solves (eight lanes per pair),
+// the overlap (one thread per pair). Between them a pair's start kind waits in
+// flags (kNoSolve: boxes apart), its start point in en, the gradients at the
+// contact point in cp_i and cp_j.
+constexpr int kNoSolve = 8;
+
+__global__ __launch_bounds__(kBlk) void k_sq_check_start(CheckArgs a) {
   const int64_t k = (int64_t)blockIdx.x * kBlk + threadIdx.x;
   if (k >= a.n) return;
   sqd::Sq A, B;
@@ -77,77 +101,110 @@ __global__ __launch_bounds__(kBlk) void k_sq_check(CheckArgs a) {
   const int state = (int)(h[0] + 0.5);
   int start = (int)(h[1] + 0.5);
   const int obb = state == 2 ? 1 : sqd::obb_intersect(A, B, start);
-  int contact = 0, iters = 0, fail = 0, fallback = 0;
-  double cp[3] = {h[2], h[3], h[4]}, fi = 0.0, fj = 0.0;
-  double en[3] = {0.0, 0.0, 0.0}, dn = 0.0, cpa[3] = {0.0, 0.0, 0.0}, cpb[3] = {0.0, 0.0, 0.0};
-  if (obb) {
-    const double ri = cbrt(A.shape[0] * A.shape[1] * A.shape[2]);
-    const double rj = cbrt(B.shape[0] * B.shape[1] * B.shape[2]);
-    const double ratio = ri / (ri + rj);
-    int fresh = state == 0;
-    if (!fresh || a.init) {
-      double est[3];
-      if (fresh) {
-        for (int c = 0; c < 3; c++) est[c] = a.init[3 * k + c];
-      } else if (a.vel && a.mass) {
-        const double *v = a.vel + 12 * k;
-        const double mi = a.mass[2 * k], mj = a.mass[2 * k + 1];
-        const double xci[3] = {cp[0] - A.center[0], cp[1] - A.center[1], cp[2] - A.center[2]};
-        const double xcj[3] = {cp[0] - B.center[0], cp[1] - B.center[1], cp[2] - B.center[2]};
-        const double *wi = v + 6, *wj = v + 9;
-        const double ri_[3] = {wi[1] * xci[2] - wi[2] * xci[1], wi[2] * xci[0] - wi[0] * xci[2],
-                               wi[0] * xci[1] - wi[1] * xci[0]};
-        const double rj_[3] = {wj[1] * xcj[2] - wj[2] * xcj[1], wj[2] * xcj[0] - wj[0] * xcj[2],
-                               wj[0] * xcj[1] - wj[1] * xcj[0]};
-        for (int c = 0; c < 3; c++) {
-          const double vi = v[c] + ri_[c], vj = v[3 + c] + rj_[c];
-          const double veff = (vi * mi + vj * mj) / (mi + mj);
-          est[c] = cp[c] + veff * a.dt;
-        }
-      } else {
-        for (int c = 0; c < 3; c++) est[c] = cp[c];
-      }
-      iters = sqd::contact_point(A, B, ratio, est, cp, fi, fj, fail, a.max_iter);
-      if (fresh) {
-        const double merit = sqd::merit_of(A.gradient, B.gradient, fi, fj);
-        if (fail || !(merit < 1e-10)) fallback = 1;
-        fresh = fallback;
-      }
+  h[1] = (double)start;
+  if (!obb) {
+    a.flags[k] = kNoSolve;
+    return;
+  }
+  const double cp[3] = {h[2], h[3], h[4]};
+  double est[3] = {cp[0], cp[1], cp[2]};
+  int kind = sqd::kStartOnly;
+  if (state == 0) {
+    kind = a.init ? sqd::kStartGiven : sqd::kStartFresh;
+    if (a.init)
+      for (int c = 0; c < 3; c++) est[c] = a.init[3 * k + c];
+  } else if (a.vel && a.mass) {
+    const double *v = a.vel + 12 * k;
+    const double mi = a.mass[2 * k], mj = a.mass[2 * k + 1];
+    const double xci[3] = {cp[0] - A.center[0], cp[1] - A.center[1], cp[2] - A.center[2]};
+    const double xcj[3] = {cp[0] - B.center[0], cp[1] - B.center[1], cp[2] - B.center[2]};
+    const double *wi = v + 6, *wj = v + 9;
+    const double ri_[3] = {wi[1] * xci[2] - wi[2] * xci[1], wi[2] * xci[0] - wi[0] * xci[2],
+                           wi[0] * xci[1] - wi[1] * xci[0]};
+    const double rj_[3] = {wj[1] * xcj[2] - wj[2] * xcj[1], wj[2] * xcj[0] - wj[0] * xcj[2],
+                           wj[0] * xcj[1] - wj[1] * xcj[0]};
+    for (int c = 0; c < 3; c++) {
+      const double vi = v[c] + ri_[c], vj = v[3 + c] + rj_[c];
+      const double veff = (vi * mi + vj * mj) / (mi + mj);
+      est[c] = cp[c] + veff * a.dt;
     }
-    if (fresh) iters += sqd::contact_point_fresh(A, B, cp, fi, fj, fail, a.max_iter);
+  }
+  a.flags[k] = kind;
+  for (int c = 0; c < 3; c++) a.en[3 * k + c] = est[c];
+}
+
+struct CheckSource {
+  const CheckArgs &a;
+  int64_t k;
+  __device__ bool next(sqd::QTask &t) {
+    do {
+      k = sqd::q_take(a.queue, a.n);
+      if (k < 0) return false;
+      t.start = a.flags[k];
+    } while (t.start == kNoSolve);
+    for (int c = 0; c < 3; c++) {
+      t.est[c] = a.en[3 * k + c];
+      t.cp[c] = a.hist[kHist * k + 2 + c];
+    }
+    return true;
+  }
+  __device__ void pose(double *p) const {
+    const double *src = ((threadIdx.x & 8) ? a.pose_b : a.pose_a) + 12 * k;
+    for (int c = 0; c < 12; c++) p[c] = src[c];
+  }
+  __device__ void put(const sqd::QResult &r, const double *cp) const {
+    if (!sqd::q_leader()) return;
+    for (int c = 0; c < 3; c++) {
+      a.point[3 * k + c] = cp[c];
+      a.cp_i[3 * k + c] = r.gA[c];
+      a.cp_j[3 * k + c] = r.gB[c];
+    }
+    a.fi[k] = r.fi;
+    a.fj[k] = r.fj;
+    a.iters[k] = r.iters;
+    a.flags[k] = r.fail | (r.fallback << 1);
+  }
+};
+
+__global__ __launch_bounds__(sqd::kGroupBlock, 2) void k_sq_check_solve(CheckArgs a) {
+  __shared__ sqd::GroupLds lds;
+  CheckSource src{a, 0};
+  sqd::q_solve_all(src, a.max_iter, lds);
+}
+
+__global__ __launch_bounds__(kBlk) void k_sq_check_finish(CheckArgs a) {
+  const int64_t k = (int64_t)blockIdx.x * kBlk + threadIdx.x;
+  if (k >= a.n) return;
+  double *h = a.hist + kHist * k;
+  double en[3] = {0.0, 0.0, 0.0}, dn = 0.0, cpa[3] = {0.0, 0.0, 0.0}, cpb[3] = {0.0, 0.0, 0.0};
+  int contact = 0;
+  if (a.flags[k] == kNoSolve) {
+    for (int c = 0; c < 3; c++) a.point[3 * k + c] = h[2 + c];
+    a.fi[k] = a.fj[k] = 0.0;
+    a.iters[k] = 0;
+    a.flags[k] = 1 << 2;
+    h[0] = 0.0;
+  } else {
+    const double cp[3] = {a.point[3 * k], a.point[3 * k + 1], a.point[3 * k + 2]};
+    const double fi = a.fi[k], fj = a.fj[k];
     contact = (fi > fj ? fi : fj) < 0.0;
     if (contact) {
-      for (int c = 0; c < 3; c++) en[c] = B.gradient[c] - A.gradient[c];
-      const double nrm = sqrt(en[0] * en[0] + en[1] * en[1] + en[2] * en[2]);
-      const double inv = nrm == 0. ? 0. : 1. / nrm;
-      for (int c = 0; c < 3; c++) en[c] *= inv;
-      const double men[3] = {-en[0], -en[1], -en[2]};
-      h[5] = sqd::line_intersection(A, cp, men, h[5], cpa);
-      h[6] = sqd::line_intersection(B, cp, en, h[6], cpb);
+      sqd::Sq A, B;
+      sqd::init(A, a.pose_a + 12 * k);
+      sqd::init(B, a.pose_b + 12 * k);
+      sqd::overlap_along_normal(A, B, cp, a.cp_i + 3 * k, a.cp_j + 3 * k, en, h[5], h[6], cpa, cpb);
       dn = fabs(h[5]) + fabs(h[6]);
-      h[0] = 2.0;
-    } else {
-      h[0] = 1.0;
     }
-    h[2] = cp[0];
-    h[3] = cp[1];
-    h[4] = cp[2];
-  } else {
-    h[0] = 0.0;
+    h[0] = contact ? 2.0 : 1.0;
+    for (int c = 0; c < 3; c++) h[2 + c] = cp[c];
   }
-  h[1] = (double)start;
   a.contact[k] = contact;
   for (int c = 0; c < 3; c++) {
     a.en[3 * k + c] = en[c];
     a.cp_i[3 * k + c] = cpa[c];
     a.cp_j[3 * k + c] = cpb[c];
-    a.point[3 * k + c] = cp[c];
   }
   a.deltan[k] = dn;
-  a.fi[k] = fi;
-  a.fj[k] = fj;
-  a.iters[k] = iters;
-  a.flags[k] = fail | (fallback << 1) | ((!obb) << 2);
 }
 
 // ---------------------------------------------------------------------------
@@ -555,15 +612,27 @@ __global__ __launch_bounds__(kBlk) void k_sample(int64_t *idx, int64_t batch, in
 // ---------------------------------------------------------------------------
 static inline unsigned nblk(int64_t n, int b) { return (unsigned)((n + b - 1) / b); }
 
+// wavefronts of a solve: the pairs spread eight to a wavefront, as far as the
+// chip holds them at once (1,024 SIMDs, two wavefronts each by registers)
+static inline unsigned solve_blocks(int64_t n) {
+  const int64_t b = (n + sqd::kGroupsPerBlock - 1) / sqd::kGroupsPerBlock;
+  return (unsigned)(b < 2048 ? b : 2048);
+}
+
 hipError_t launch_solve(const SolveArgs &a, hipStream_t s) {
   if (a.n <= 0) return hipSuccess;
-  hipLaunchKernelGGL(k_sq_solve, dim3(nblk(a.n, kBlk)), dim3(kBlk), 0, s, a);
+  hipLaunchKernelGGL(k_zero_queue, dim3(1), dim3(1), 0, s, a.queue);
+  hipLaunchKernelGGL(k_sq_solve, dim3(solve_blocks(a.n)), dim3(sqd::kGroupBlock), 0, s, a);
+  if (a.polish > 0) hipLaunchKernelGGL(k_sq_polish, dim3(nblk(a.n, kBlk)), dim3(kBlk), 0, s, a);
   return hipGetLastError();
 }
 
 hipError_t launch_check(const CheckArgs &a, hipStream_t s) {
   if (a.n <= 0) return hipSuccess;
-  hipLaunchKernelGGL(k_sq_check, dim3(nblk(a.n, kBlk)), dim3(kBlk), 0, s, a);
+  hipLaunchKernelGGL(k_sq_check_start, dim3(nblk(a.n, kBlk)), dim3(kBlk), 0, s, a);
+  hipLaunchKernelGGL(k_zero_queue, dim3(1), dim3(1), 0, s, a.queue);
+  hipLaunchKernelGGL(k_sq_check_solve, dim3(solve_blocks(a.n)), dim3(sqd::kGroupBlock), 0, s, a);
+  hipLaunchKernelGGL(k_sq_check_finish, dim3(nblk(a.n, kBlk)), dim3(kBlk), 0, s, a);
   return hipGetLastError();
 }
 

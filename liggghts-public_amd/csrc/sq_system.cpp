@@ -22,6 +22,7 @@ struct dem_sq_handle {
   double *pose_a = nullptr, *pose_b = nullptr, *init = nullptr, *point = nullptr, *fi = nullptr,
          *fj = nullptr;
   int *iters = nullptr, *flags = nullptr;
+  unsigned *queue = nullptr;  // next pair of a running solve
   float *X = nullptr, *Y = nullptr, *T = nullptr;  // network inputs / outputs / targets of the pairs
   bool have_fresh = false;                         // point holds a fresh (plain) solve
   // contact detection buffers, allocated with the pair set on first use
@@ -178,6 +179,7 @@ int dem_sq_set_pairs(dem_sq_handle *h, int64_t n, const double *pose_a, const do
       (rc = A((void **)&h->init, sizeof(double) * 3 * N)) || (rc = A((void **)&h->point, sizeof(double) * 3 * N)) ||
       (rc = A((void **)&h->fi, sizeof(double) * N)) || (rc = A((void **)&h->fj, sizeof(double) * N)) ||
       (rc = A((void **)&h->iters, sizeof(int) * N)) || (rc = A((void **)&h->flags, sizeof(int) * N)) ||
+      (rc = A((void **)&h->queue, sizeof(unsigned))) ||
       (rc = A((void **)&h->X, sizeof(float) * sqk::kIn * N)) || (rc = A((void **)&h->Y, sizeof(float) * sqk::kOut * N)) ||
       (rc = A((void **)&h->T, sizeof(float) * sqk::kOut * N)))
     return rc;
@@ -221,6 +223,7 @@ int dem_sq_solve(dem_sq_handle *h, int start, const double *init, int polish) {
   a.fj = h->fj;
   a.iters = h->iters;
   a.fail = h->flags;
+  a.queue = h->queue;
   SQCHK(h, sqk::launch_solve(a, h->stream));
   SQCHK(h, hipEventRecord(h->ev[2], h->stream));
   SQCHK(h, hipEventSynchronize(h->ev[2]));
@@ -299,6 +302,7 @@ int dem_sq_check(dem_sq_handle *h, int start, double dt, const double *vel, cons
   a.fj = h->fj;
   a.iters = h->iters;
   a.flags = h->flags;
+  a.queue = h->queue;
   SQCHK(h, sqk::launch_check(a, h->stream));
   SQCHK(h, hipEventRecord(h->ev[2], h->stream));
   SQCHK(h, hipEventSynchronize(h->ev[2]));

@@ -50,7 +50,15 @@ struct Dev {
   const double *init;
   const int *fresh_idx;
   int max_iter;
+  // this step's solves: the pairs whose contact point is wanted and how each
+  // starts, per pair the start point and then the result (contact point, shape
+  // function values, gradients), its iterations and whether the start fell back
+  int *solve_list, *solve_kind, *solve_iters;
+  double *sol;  // [np][kSol]
+  unsigned *solve_count;  // [0] entries of solve_list, [1] the next to be taken
 };
+
+constexpr int kSol = 11;
 
 struct Grid {
   int nc[3];
@@ -88,6 +96,7 @@ hipError_t launch_accumulate(const unsigned long long *stats, unsigned long long
 // pairs far apart last step whose OBBs overlap: compact list and their poses
 hipError_t launch_fresh_scan(const Dev &d, int *fresh_idx, int *fresh_count, double *pose_a, double *pose_b,
                              hipStream_t s);
+// contact detection and the force records, in three launches
 hipError_t launch_pairs(const Dev &d, int shearupdate, hipStream_t s);
 // sums pair records, adds plane walls and gravity, and (integrate) the final half step
 hipError_t launch_gather(const Dev &d, int shearupdate, int integrate, hipStream_t s);

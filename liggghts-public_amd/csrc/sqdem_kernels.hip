@@ -13,8 +13,11 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <algorithm>
+
 #include "dem_device.h"
 #include "sq_device.h"
+#include "sq_group.h"
 #include "sqdem_kernels.h"
 
 namespace sqdk {
@@ -485,45 +488,56 @@ __device__ __forceinline__ void contact_force(const Dev &d, int itype, int jtype
   }
 }
 
-// PairGran compute loop body (pair_gran_base.h:255-430) for one pair with the
-// superquadric surface model: checkSurfaceIntersect
-// (surface_model_superquadric.h:108-205) on overlapping bounding spheres, the
-// force chain on intersecting surfaces, surfacesClose (zero shear) otherwise
-__global__ __launch_bounds__(kBlk) void k_pairs(Dev d, int shearupdate) {
+// sums a counter over the wavefront and adds it with one atomic
+__device__ __forceinline__ void wave_count(unsigned long long *stat, unsigned v) {
+  for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
+  if ((threadIdx.x & 63) == 0 && v) atomicAdd(stat, (unsigned long long)v);
+}
+
+// PairGran compute loop body (pair_gran_base.h:255-430) with the superquadric
+// surface model: checkSurfaceIntersect (surface_model_superquadric.h:108-205)
+// on overlapping bounding spheres, the force chain on intersecting surfaces,
+// surfacesClose (zero shear) otherwise. Three launches: k_pair_start (one
+// thread per pair) runs the box test, finishes the pairs apart and lists the
+// others with their start points; k_pair_solve (eight lanes per pair) finds
+// their contact points; k_pair_finish (one thread per listed pair) the overlap
+// and the forces. One launch with a thread per pair lasted as long as its
+// slowest lane's solve, 18 us an iteration (sq_group.h).
+__global__ __launch_bounds__(kBlk) void k_pair_start(Dev d) {
   const int64_t p = (int64_t)blockIdx.x * kBlk + threadIdx.x;
-  if (p >= d.np) return;
-  double *rec = d.rec + (size_t)kRec * p;
-  double out[kRec];
-  for (int k = 0; k < kRec; k++) out[k] = 0.0;
-  const int i = d.pi[p], j = d.pj[p];
-  double xj[3], del[3];
-  image_of(d, i, j, xj, del);
-  const double rsq = del[0] * del[0] + del[1] * del[1] + del[2] * del[2];
-  const double radsum = d.rb[i] + d.rb[j];
-  if (rsq < radsum * radsum) {
-    double *h = d.hist + (size_t)kHist * p;
-    double poseA[12], poseB[12];
-    load_pose(d, i, d.x + 3 * i, poseA);
-    load_pose(d, j, xj, poseB);
-    sqd::Sq A, B;
-    sqd::init(A, poseA);
-    sqd::init(B, poseB);
-    const int state = (int)(h[0] + 0.5);
-    int start = (int)(h[1] + 0.5);
-    const int obb = state == 2 ? 1 : sqd::obb_intersect(A, B, start);
-    int contact = 0, iters = 0, fail = 0, fallback = 0;
-    double cp[3] = {h[2], h[3], h[4]}, fi = 0.0, fj = 0.0, en[3] = {0.0, 0.0, 0.0}, dn = 0.0;
-    if (obb) {
-      const double ri = cbrt(A.shape[0] * A.shape[1] * A.shape[2]);
-      const double rj = cbrt(B.shape[0] * B.shape[1] * B.shape[2]);
-      const double ratio = ri / (ri + rj);
-      int fresh = state == 0;
-      const int slot = (fresh && d.init) ? d.fresh_idx[p] : -1;
-      if (!fresh || slot >= 0) {
-        double est[3];
+  bool checked = false, solve = false, fresh = false;
+  if (p < d.np) {
+    const int i = d.pi[p], j = d.pj[p];
+    double xj[3], del[3];
+    image_of(d, i, j, xj, del);
+    const double rsq = del[0] * del[0] + del[1] * del[1] + del[2] * del[2];
+    const double radsum = d.rb[i] + d.rb[j];
+    checked = rsq < radsum * radsum;
+    if (checked) {
+      double *h = d.hist + (size_t)kHist * p;
+      double poseA[12], poseB[12];
+      load_pose(d, i, d.x + 3 * i, poseA);
+      load_pose(d, j, xj, poseB);
+      sqd::Sq A, B;
+      sqd::init(A, poseA);
+      sqd::init(B, poseB);
+      const int state = (int)(h[0] + 0.5);
+      int start = (int)(h[1] + 0.5);
+      solve = state == 2 || sqd::obb_intersect(A, B, start);
+      h[1] = (double)start;
+      if (solve) {
+        fresh = state == 0;
+        const int slot = (fresh && d.init) ? d.fresh_idx[p] : -1;
+        int kind = sqd::kStartOnly;
+        double est[3] = {0.0, 0.0, 0.0};
         if (fresh) {
-          for (int c = 0; c < 3; c++) est[c] = d.init[3 * (size_t)slot + c];
+          kind = slot >= 0 ? sqd::kStartGiven : sqd::kStartFresh;
+          if (slot >= 0)
+            for (int c = 0; c < 3; c++) est[c] = d.init[3 * (size_t)slot + c];
         } else {
+          // calc_contact_point_using_prev_step: the last point moved by the
+          // mass-weighted contact velocity
+          const double cp[3] = {h[2], h[3], h[4]};
           const double mi = d.mass[i], mj = d.mass[j];
           const double *wi = d.w + 3 * i, *wj = d.w + 3 * j;
           const double xci[3] = {cp[0] - A.center[0], cp[1] - A.center[1], cp[2] - A.center[2]};
@@ -537,58 +551,127 @@ __global__ __launch_bounds__(kBlk) void k_pairs(Dev d, int shearupdate) {
             est[c] = cp[c] + veff * d.dt;
           }
         }
-        iters = sqd::contact_point(A, B, ratio, est, cp, fi, fj, fail, d.max_iter);
-        if (fresh) {
-          const double merit = sqd::merit_of(A.gradient, B.gradient, fi, fj);
-          if (fail || !(merit < 1e-10)) fallback = 1;
-          fresh = fallback;
-        }
+        d.solve_kind[p] = kind;
+        for (int c = 0; c < 3; c++) d.sol[(size_t)kSol * p + c] = est[c];
+      } else {
+        h[0] = 0.0;
+        h[7] = h[8] = h[9] = 0.0;
       }
-      if (fresh) iters += sqd::contact_point_fresh(A, B, cp, fi, fj, fail, d.max_iter);
-      if (state == 0) {
-        atomicAdd(&d.stats[kStatFresh], 1ull);
-        atomicAdd(&d.stats[kStatFreshIters], (unsigned long long)iters);
-        if (fallback) atomicAdd(&d.stats[kStatFallback], 1ull);
+    }
+    if (!solve) {
+      double *rec = d.rec + (size_t)kRec * p;
+      for (int k = 0; k < kRec; k++) rec[k] = 0.0;
+    }
+  }
+  // the wavefront's pairs join the list together
+  const unsigned long long m = __ballot(solve);
+  unsigned base = 0;
+  if (m != 0ull) {
+    const int lead = __ffsll((long long)m) - 1;
+    if ((int)(threadIdx.x & 63) == lead) base = atomicAdd(d.solve_count, (unsigned)__popcll(m));
+    base = __shfl(base, lead, 64);
+  }
+  if (solve) d.solve_list[base + __popcll(m & ((1ull << (threadIdx.x & 63)) - 1ull))] = (int)p;
+  wave_count(&d.stats[kStatChecked], checked);
+  wave_count(&d.stats[kStatFresh], fresh);
+}
+
+struct PairSource {
+  const Dev &d;
+  const int64_t n;
+  int64_t p;
+  __device__ bool next(sqd::QTask &t) {
+    const int64_t k = sqd::q_take(d.solve_count + 1, n);
+    if (k < 0) return false;
+    p = d.solve_list[k];
+    t.start = d.solve_kind[p];
+    for (int c = 0; c < 3; c++) {
+      t.est[c] = d.sol[(size_t)kSol * p + c];
+      t.cp[c] = d.hist[(size_t)kHist * p + 2 + c];
+    }
+    return true;
+  }
+  __device__ void pose(double *out) const {
+    const int i = d.pi[p], j = d.pj[p];
+    double xj[3], del[3];
+    image_of(d, i, j, xj, del);
+    if (threadIdx.x & 8)
+      load_pose(d, j, xj, out);
+    else
+      load_pose(d, i, d.x + 3 * i, out);
+  }
+  __device__ void put(const sqd::QResult &r, const double *cp) const {
+    if (!sqd::q_leader()) return;
+    double *o = d.sol + (size_t)kSol * p;
+    for (int c = 0; c < 3; c++) {
+      o[c] = cp[c];
+      o[5 + c] = r.gA[c];
+      o[8 + c] = r.gB[c];
+    }
+    o[3] = r.fi;
+    o[4] = r.fj;
+    d.solve_iters[p] = r.iters * 2 + r.fallback;
+  }
+};
+
+__global__ __launch_bounds__(sqd::kGroupBlock, 2) void k_pair_solve(Dev d) {
+  __shared__ sqd::GroupLds lds;
+  PairSource src{d, (int64_t)d.solve_count[0], 0};
+  sqd::q_solve_all(src, d.max_iter, lds);
+}
+
+__global__ __launch_bounds__(kBlk) void k_pair_finish(Dev d, int shearupdate) {
+  const unsigned n = d.solve_count[0];
+  for (unsigned k0 = blockIdx.x * kBlk; k0 < n; k0 += gridDim.x * kBlk) {
+    const unsigned k = k0 + threadIdx.x;
+    unsigned iters = 0, fresh_iters = 0, fallback = 0, contact = 0;
+    if (k < n) {
+      const int64_t p = d.solve_list[k];
+      const int i = d.pi[p], j = d.pj[p];
+      double xj[3], del[3];
+      image_of(d, i, j, xj, del);
+      double *h = d.hist + (size_t)kHist * p;
+      const double *o = d.sol + (size_t)kSol * p;
+      const double cp[3] = {o[0], o[1], o[2]}, fi = o[3], fj = o[4];
+      double out[kRec];
+      for (int q = 0; q < kRec; q++) out[q] = 0.0;
+      iters = (unsigned)d.solve_iters[p] >> 1;
+      if (d.solve_kind[p] != sqd::kStartOnly) {
+        fresh_iters = iters;
+        fallback = (unsigned)d.solve_iters[p] & 1u;
       }
       contact = (fi > fj ? fi : fj) < 0.0;
       if (contact) {
-        for (int c = 0; c < 3; c++) en[c] = B.gradient[c] - A.gradient[c];
-        const double nrm = sqrt(en[0] * en[0] + en[1] * en[1] + en[2] * en[2]);
-        const double inv = nrm == 0. ? 0. : 1. / nrm;
-        for (int c = 0; c < 3; c++) en[c] *= inv;
-        const double men[3] = {-en[0], -en[1], -en[2]};
-        double cpa[3], cpb[3];
-        h[5] = sqd::line_intersection(A, cp, men, h[5], cpa);
-        h[6] = sqd::line_intersection(B, cp, en, h[6], cpb);
-        dn = fabs(h[5]) + fabs(h[6]);
+        double poseA[12], poseB[12], en[3], cpa[3], cpb[3];
+        load_pose(d, i, d.x + 3 * i, poseA);
+        load_pose(d, j, xj, poseB);
+        sqd::Sq A, B;
+        sqd::init(A, poseA);
+        sqd::init(B, poseB);
+        sqd::overlap_along_normal(A, B, cp, o + 5, o + 8, en, h[5], h[6], cpa, cpb);
+        const double dn = fabs(h[5]) + fabs(h[6]);
         h[0] = 2.0;
+        d.flag[p] = 1;
+        const double rvi = d.rv[i], rvj = d.rv[j];
+        const double mi = d.mass[i], mj = d.mass[j];
+        const double xci[3] = {cp[0] - d.x[3 * i], cp[1] - d.x[3 * i + 1], cp[2] - d.x[3 * i + 2]};
+        const double xcj[3] = {cp[0] - xj[0], cp[1] - xj[1], cp[2] - xj[2]};
+        contact_force(d, d.type[i], d.type[j], 0, rvi * rvj / (rvi + rvj), mi * mj / (mi + mj), dn, en,
+                      d.v + 3 * i, d.v + 3 * j, d.w + 3 * i, d.w + 3 * j, xci, xcj, shearupdate, h + 7, out,
+                      out + 3, out + 6);
       } else {
         h[0] = 1.0;
+        h[7] = h[8] = h[9] = 0.0;
       }
-      h[2] = cp[0];
-      h[3] = cp[1];
-      h[4] = cp[2];
-    } else {
-      h[0] = 0.0;
+      for (int c = 0; c < 3; c++) h[2 + c] = cp[c];
+      double *rec = d.rec + (size_t)kRec * p;
+      for (int q = 0; q < kRec; q++) rec[q] = out[q];
     }
-    h[1] = (double)start;
-    atomicAdd(&d.stats[kStatChecked], 1ull);
-    if (iters) atomicAdd(&d.stats[kStatNewton], (unsigned long long)iters);
-    if (contact) {
-      d.flag[p] = 1;
-      atomicAdd(&d.stats[kStatPairTouch], 1ull);
-      const double rvi = d.rv[i], rvj = d.rv[j];
-      const double mi = d.mass[i], mj = d.mass[j];
-      const double xci[3] = {cp[0] - d.x[3 * i], cp[1] - d.x[3 * i + 1], cp[2] - d.x[3 * i + 2]};
-      const double xcj[3] = {cp[0] - xj[0], cp[1] - xj[1], cp[2] - xj[2]};
-      contact_force(d, d.type[i], d.type[j], 0, rvi * rvj / (rvi + rvj), mi * mj / (mi + mj), dn, en,
-                    d.v + 3 * i, d.v + 3 * j, d.w + 3 * i, d.w + 3 * j, xci, xcj, shearupdate, h + 7, out,
-                    out + 3, out + 6);
-    } else {
-      h[7] = h[8] = h[9] = 0.0;
-    }
+    wave_count(&d.stats[kStatNewton], iters);
+    wave_count(&d.stats[kStatFreshIters], fresh_iters);
+    wave_count(&d.stats[kStatFallback], fallback);
+    wave_count(&d.stats[kStatPairTouch], contact);
   }
-  for (int k = 0; k < kRec; k++) rec[k] = out[k];
 }
 
 // Superquadric::plane_intersection (superquadric.cpp:440-507): the point of
@@ -828,7 +911,13 @@ hipError_t launch_fresh_scan(const Dev &d, int *fresh_idx, int *fresh_count, dou
 
 hipError_t launch_pairs(const Dev &d, int shearupdate, hipStream_t s) {
   if (d.np <= 0) return hipSuccess;
-  hipLaunchKernelGGL(k_pairs, dim3(nblk(d.np, kBlk)), dim3(kBlk), 0, s, d, shearupdate);
+  hipLaunchKernelGGL(k_zero_int, dim3(1), dim3(kBlk), 0, s, (int *)d.solve_count, 2);
+  hipLaunchKernelGGL(k_pair_start, dim3(nblk(d.np, kBlk)), dim3(kBlk), 0, s, d);
+  // the lists' lengths stay on the device: as many blocks as could be needed,
+  // up to what the chip holds at once
+  hipLaunchKernelGGL(k_pair_solve, dim3(std::min(nblk(d.np, sqd::kGroupsPerBlock), 2048)), dim3(sqd::kGroupBlock),
+                     0, s, d);
+  hipLaunchKernelGGL(k_pair_finish, dim3(std::min(nblk(d.np, kBlk), 1024)), dim3(kBlk), 0, s, d, shearupdate);
   return hipGetLastError();
 }
 

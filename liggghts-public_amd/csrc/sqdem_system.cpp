@@ -63,14 +63,14 @@ struct dem_sqdem_handle {
   int *count = nullptr, *scan_tmp = nullptr, *rcount = nullptr, *rfirst = nullptr, *rfill = nullptr;
   int *overflow = nullptr, *dflag = nullptr;
   int pair_cap = 0;
-  int *rlist = nullptr, *fresh_idx = nullptr;
-  double *rec = nullptr;
+  int *rlist = nullptr, *fresh_idx = nullptr, *solve_list = nullptr, *solve_kind = nullptr, *solve_iters = nullptr;
+  double *rec = nullptr, *sol = nullptr;
   std::vector<void *> pair_allocs;
   unsigned long long *stats = nullptr, *totals = nullptr;
   int *hflag = nullptr;  // pinned
   // warm start
   dem_sq_handle *net = nullptr;
-  int *fresh_count = nullptr;
+  int *fresh_count = nullptr;  // [0] listed fresh pairs; [2], [3] the step's solves (Dev::solve_count)
   int64_t fresh_cap = 0;
   double *fpa = nullptr, *fpb = nullptr, *finit = nullptr;
   float *fX = nullptr, *fY = nullptr;
@@ -272,6 +272,11 @@ sqdk::Dev make_dev(dem_sqdem_handle *h) {
   d.stats = h->stats;
   d.init = nullptr;
   d.fresh_idx = h->fresh_idx;
+  d.solve_list = h->solve_list;
+  d.solve_kind = h->solve_kind;
+  d.solve_iters = h->solve_iters;
+  d.sol = h->sol;
+  d.solve_count = (unsigned *)h->fresh_count + 2;
   d.max_iter = 100000;  // Niter of calc_contact_point (math_extra_liggghts_superquadric.cpp:856)
   return d;
 }
@@ -304,6 +309,10 @@ int ensure_pair_arrays(dem_sqdem_handle *h, int np) {
   int rc;
   if ((rc = dalloc(h, h->pair_allocs, (void **)&h->rlist, sizeof(int) * cap)) ||
       (rc = dalloc(h, h->pair_allocs, (void **)&h->fresh_idx, sizeof(int) * cap)) ||
+      (rc = dalloc(h, h->pair_allocs, (void **)&h->solve_list, sizeof(int) * cap)) ||
+      (rc = dalloc(h, h->pair_allocs, (void **)&h->solve_kind, sizeof(int) * cap)) ||
+      (rc = dalloc(h, h->pair_allocs, (void **)&h->solve_iters, sizeof(int) * cap)) ||
+      (rc = dalloc(h, h->pair_allocs, (void **)&h->sol, sizeof(double) * sqdk::kSol * (size_t)cap)) ||
       (rc = dalloc(h, h->pair_allocs, (void **)&h->rec, sizeof(double) * sqdk::kRec * (size_t)cap)))
     return rc;
   h->pair_cap = cap;
