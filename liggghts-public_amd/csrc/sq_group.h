@@ -241,9 +241,12 @@ __device__ __forceinline__ void q_direction(int c, const double *jc, const doubl
     }
     invert = fabs(det4(J4)) > 1.0;
     if (!invert) {
-      double d0[4];
+      // copies: arrays whose address leaves the function live in scratch memory
+      double Fc[4], d0[4], d1[4];
+      cp4(Fc, F);
       cp4(d0, delta);
-      gmres44_cold(J4, F, d0, delta);
+      gmres44_cold(J4, Fc, d0, d1);
+      cp4(delta, d1);
     }
   }
   if (invert) {
