@@ -297,7 +297,19 @@ struct WallLocalArgs {
   int ncol;
 };
 
+// the state in the caller's order: out[q] (x, v, omega, f, torque; null: not
+// wanted) are [n][3] doubles; *bad is set when orig holds an index outside [0, n)
+struct ExportArgs {
+  int n, cap, mixed;
+  StateBuf st;
+  const int *orig;
+  const double *fout;
+  double *out[5];
+  int *bad;
+};
+
 // launchers (dem_kernels.hip)
+hipError_t launch_export(const ExportArgs &a, hipStream_t s);
 hipError_t launch_rebuild(const RebuildArgs &a, hipStream_t s);
 hipError_t launch_step(const StepArgs &a, hipStream_t s);
 hipError_t launch_initial(const StepArgs &a, hipStream_t s);

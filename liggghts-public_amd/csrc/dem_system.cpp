@@ -126,6 +126,8 @@ struct dem_handle {
   bool setup_done = false;
   bool can_continue = false;  // fout holds the last force pass in the current order
   double *xhold = nullptr, *fout = nullptr;
+  double *export_buf = nullptr;  // dem_get_state: the arrays in caller order, then the flag
+  int64_t export_n = 0;          // particles it has room for, five arrays each
   double rmax = 0.0;
   double rmax_future = 0.0;  // dem_set_max_radius: particles still to come
   // particles waiting to join at the next run's first step (dem_insert_particles)
@@ -234,6 +236,8 @@ void free_particles(dem_handle *h) {
     h->lst[b] = ListBuf{};
   }
   h->xhold = h->fout = nullptr;
+  h->export_buf = nullptr;
+  h->export_n = 0;
   h->d_tri_buf[0] = h->d_tri_buf[1] = nullptr;
   h->d_node_last = nullptr;
   h->d_motion = nullptr;
@@ -1988,58 +1992,38 @@ int dem_get_box(dem_handle *h, double *boxlo, double *boxhi) {
 int dem_get_state(dem_handle *h, double *x, double *v, double *omega, double *f, double *torque) {
   if (!h) return DEM_ERR_ARG;
   if (h->n <= 0) return DEM_OK;  // an empty system (particles still to be inserted): nothing to copy
-  HIPCHK(h, hipStreamSynchronize(h->stream));
+  HIPCHK(h, hipSetDevice(h->p.device));
   const int64_t n = h->n;
-  const size_t cap = (size_t)h->cap;
-  std::vector<double4> pos(n), vel(n);
-  std::vector<int> orig(n);
-  const StateBuf &s = h->st[h->cur_st];
-  HIPCHK(h, hipMemcpy(pos.data(), s.pos, sizeof(double4) * n, hipMemcpyDeviceToHost));
-  HIPCHK(h, hipMemcpy(vel.data(), s.vel, sizeof(double4) * n, hipMemcpyDeviceToHost));
-  HIPCHK(h, hipMemcpy(orig.data(), h->aux[h->cur_aux].orig, sizeof(int) * n, hipMemcpyDeviceToHost));
-  std::vector<double> w(3 * n);
-  if (h->mixed) {
-    std::vector<float4> ww(n);
-    HIPCHK(h, hipMemcpy(ww.data(), s.omg, sizeof(float4) * n, hipMemcpyDeviceToHost));
-    for (int64_t i = 0; i < n; i++) {
-      w[3 * i] = ww[i].x;
-      w[3 * i + 1] = ww[i].y;
-      w[3 * i + 2] = ww[i].z;
-    }
-  } else {
-    std::vector<double4> ww(n);
-    HIPCHK(h, hipMemcpy(ww.data(), s.omg, sizeof(double4) * n, hipMemcpyDeviceToHost));
-    for (int64_t i = 0; i < n; i++) {
-      w[3 * i] = ww[i].x;
-      w[3 * i + 1] = ww[i].y;
-      w[3 * i + 2] = ww[i].z;
-    }
+  if (n > h->export_n) {
+    HIPCHK(h, hipStreamSynchronize(h->stream));
+    dfree(h, h->export_buf);
+    h->export_buf = nullptr;
+    h->export_n = 0;
+    const int64_t room = std::max<int64_t>(n, h->cap);
+    int rc = dalloc(h, (void **)&h->export_buf, sizeof(double) * (15 * (size_t)room + 1));
+    if (rc) return rc;
+    h->export_n = room;
   }
-  std::vector<double> ft;
-  if (f || torque) {
-    ft.resize(6 * cap);
-    HIPCHK(h, hipMemcpy(ft.data(), h->fout, sizeof(double) * 6 * cap, hipMemcpyDeviceToHost));
-  }
-  for (int64_t i = 0; i < n; i++) {
-    const int o = orig[i];
-    if (o < 0 || o >= n) return fail(h, DEM_ERR_STATE, "corrupt particle index");
-    if (x) {
-      x[3 * o] = pos[i].x;
-      x[3 * o + 1] = pos[i].y;
-      x[3 * o + 2] = pos[i].z;
-    }
-    if (v) {
-      v[3 * o] = vel[i].x;
-      v[3 * o + 1] = vel[i].y;
-      v[3 * o + 2] = vel[i].z;
-    }
-    if (omega)
-      for (int d = 0; d < 3; d++) omega[3 * o + d] = w[3 * i + d];
-    if (f)
-      for (int d = 0; d < 3; d++) f[3 * o + d] = ft[d * cap + i];
-    if (torque)
-      for (int d = 0; d < 3; d++) torque[3 * o + d] = ft[(3 + d) * cap + i];
-  }
+  // reordered on the device, so each array is one contiguous copy
+  dem::ExportArgs e{};
+  e.n = (int)n;
+  e.cap = h->cap;
+  e.mixed = h->mixed ? 1 : 0;
+  e.st = h->st[h->cur_st];
+  e.orig = h->aux[h->cur_aux].orig;
+  e.fout = h->fout;
+  double *dst[5] = {x, v, omega, f, torque};
+  for (int q = 0; q < 5; q++) e.out[q] = dst[q] ? h->export_buf + 3 * (size_t)h->export_n * q : nullptr;
+  e.bad = (int *)(h->export_buf + 15 * (size_t)h->export_n);
+  HIPCHK(h, dem::launch_export(e, h->stream));
+  int bad = 0;
+  HIPCHK(h, hipMemcpyAsync(&bad, e.bad, sizeof(int), hipMemcpyDeviceToHost, h->stream));
+  HIPCHK(h, hipStreamSynchronize(h->stream));
+  if (bad) return fail(h, DEM_ERR_STATE, "corrupt particle index");
+  for (int q = 0; q < 5; q++)
+    if (dst[q])
+      HIPCHK(h, hipMemcpyAsync(dst[q], e.out[q], sizeof(double) * 3 * (size_t)n, hipMemcpyDeviceToHost, h->stream));
+  HIPCHK(h, hipStreamSynchronize(h->stream));
   return DEM_OK;
 }
 
