@@ -21,7 +21,10 @@ constexpr int kNumParams = kOffB3 + kOut;
 
 struct NetDev {
   float *params, *m, *v;            // FP32 master parameters and Adam moments
-  unsigned short *w1b, *w2b, *w3b;  // BF16 weights, [kInPad][kHid], [kHid][kHid], [kHid][kOutPad]
+  // BF16 weights as the matrix cores' A operands, one 8-byte piece per lane and
+  // 16 x 16 tile (frag_at): W^T of each layer (forward), W2 and W3 (backward);
+  // inputs padded to kInPad, outputs to kOutPad
+  unsigned short *w1f, *w2f, *w3f, *w2t, *w3t;
   float *b1, *b2, *b3;              // FP32 biases, b3 padded to kOutPad
 };
 
@@ -70,23 +73,37 @@ __device__ __forceinline__ unsigned short pack_bf16(float f) {
   return (unsigned short)(u >> 16);
 }
 
-// parameter i -> the copy the matrix cores read
+// where element (row, k) of an A operand of `ksteps` tiles along k sits: lane
+// (k % 16 / 4) * 16 + row % 16 of tile (row / 16, k / 16), slot k % 4
+__host__ __device__ constexpr int frag_at(int row, int k, int ksteps) {
+  return (((row / 16) * ksteps + k / 16) * 64 + (k % 16) / 4 * 16 + row % 16) * 4 + k % 4;
+}
+
+// parameter i -> the copies the matrix cores read
 __device__ __forceinline__ void write_packed(const NetDev &net, int i, float p) {
   if (i < kOffB1) {
-    net.w1b[(i / kHid) * kHid + i % kHid] = pack_bf16(p);
+    net.w1f[frag_at(i % kHid, i / kHid, kInPad / 16)] = pack_bf16(p);
   } else if (i < kOffW2) {
     net.b1[i - kOffB1] = p;
   } else if (i < kOffB2) {
-    net.w2b[i - kOffW2] = pack_bf16(p);
+    const int k = (i - kOffW2) / kHid, f = (i - kOffW2) % kHid;
+    net.w2f[frag_at(f, k, kHid / 16)] = net.w2t[frag_at(k, f, kHid / 16)] = pack_bf16(p);
   } else if (i < kOffW3) {
     net.b2[i - kOffB2] = p;
   } else if (i < kOffB3) {
-    const int k = i - kOffW3;
-    net.w3b[(k / kOut) * kOutPad + k % kOut] = pack_bf16(p);
+    const int k = (i - kOffW3) / kOut, f = (i - kOffW3) % kOut;
+    net.w3f[frag_at(f, k, kHid / 16)] = net.w3t[frag_at(k, f, kOutPad / 16)] = pack_bf16(p);
   } else {
     net.b3[i - kOffB3] = p;
   }
 }
+
+// the rows of X / T a batch consists of: 0 .. batch-1, or (n > 0) drawn
+// uniformly with replacement from [0, n)
+struct RowPick {
+  int64_t n;
+  uint64_t seed;
+};
 
 hipError_t launch_solve(const SolveArgs &a, hipStream_t s);
 hipError_t launch_check(const CheckArgs &a, hipStream_t s);
@@ -97,13 +114,11 @@ hipError_t launch_to_target(const double *pa, const double *pb, int64_t n, const
                             hipStream_t s);
 hipError_t launch_mlp_forward(const NetDev &net, const float *X, int64_t n, float *Y, hipStream_t s);
 int grad_blocks(int64_t batch);
-// idx: the batch's rows of X / T, or null for rows 0 .. batch-1
-hipError_t launch_mlp_grad(const NetDev &net, const float *X, const float *T, const int64_t *idx,
+hipError_t launch_mlp_grad(const NetDev &net, const float *X, const float *T, const RowPick &pick,
                            int64_t batch, float *part, float *loss_part, hipStream_t s);
 hipError_t launch_mlp_adam(const NetDev &net, const float *part, int nparts, float *grad, const AdamArgs &ad,
                            hipStream_t s);
 hipError_t launch_mlp_pack(const NetDev &net, hipStream_t s);
-hipError_t launch_sample(int64_t *idx, int64_t batch, int64_t n, uint64_t seed, hipStream_t s);
 
 // the allocation-free gradient's workspace (a file-scope device array in
 // sq_kernels.hip): batches up to kGradScratchMaxBatch samples, devices

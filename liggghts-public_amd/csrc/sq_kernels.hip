@@ -276,316 +276,273 @@ __global__ __launch_bounds__(kBlk) void k_sq_frame(const double *pa, const doubl
 // v_mfma_f32_16x16x16_bf16 lane layout (64 lanes, l = lane, r = l % 16,
 // q = l / 16): A (16 x 16, M x K) element A[r][4q + j] in slot j of the lane's
 // bf16x4; B (K x N) element B[4q + j][r]; the FP32 result D[4q + j][r] in
-// slot j. One wavefront owns a tile of 16 samples.
+// slot j. One wavefront owns a tile of 16 samples and computes every layer
+// transposed, H^T = W^T X^T: a layer's result (feature 4q + j of sample r) is
+// then the next layer's B operand as it stands, so activations and deltas pass
+// from product to product in registers, and the weights are A operands read
+// from the L2 as the lane's own 8 bytes. Only the weight gradients, whose
+// products run over the samples, take their operands through LDS.
 // ---------------------------------------------------------------------------
 __device__ __forceinline__ unsigned short to_bf16(float f) { return pack_bf16(f); }
-
-__device__ __forceinline__ float from_bf16(unsigned short h) { return __uint_as_float((unsigned int)h << 16); }
 
 __device__ __forceinline__ floatx4 mfma(bf16x4 a, bf16x4 b, floatx4 c) {
   return __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, b, c, 0, 0, 0);
 }
 
-// A operand: rows r0.., columns k0.. of a row-major bf16 matrix (leading dim ld)
-__device__ __forceinline__ bf16x4 ld_a(const unsigned short *M, int ld, int r0, int k0) {
-  const int l = threadIdx.x & 63;
-  const unsigned short *p = M + (r0 + (l & 15)) * ld + k0 + 4 * (l >> 4);
-  bf16x4 v;
-  v[0] = (short)p[0];
-  v[1] = (short)p[1];
-  v[2] = (short)p[2];
-  v[3] = (short)p[3];
-  return v;
+__device__ __forceinline__ bf16x4 pack4(const floatx4 &v) {
+  bf16x4 o;
+  for (int j = 0; j < 4; j++) o[j] = (short)to_bf16(v[j]);
+  return o;
 }
 
-// A operand of a transposed matrix: A[m][k] = M[k][m]
-__device__ __forceinline__ bf16x4 ld_at(const unsigned short *M, int ld, int m0, int k0) {
-  const int l = threadIdx.x & 63;
-  const int m = m0 + (l & 15), k = k0 + 4 * (l >> 4);
-  bf16x4 v;
-  v[0] = (short)M[(k + 0) * ld + m];
-  v[1] = (short)M[(k + 1) * ld + m];
-  v[2] = (short)M[(k + 2) * ld + m];
-  v[3] = (short)M[(k + 3) * ld + m];
-  return v;
+// A operand: tile t of a packed weight array
+__device__ __forceinline__ bf16x4 ld_w(const unsigned short *w, int t) {
+  return *(const bf16x4 *)(w + ((size_t)t * 64 + (threadIdx.x & 63)) * 4);
 }
 
-// B operand: B[k][n] of a row-major bf16 matrix
-__device__ __forceinline__ bf16x4 ld_b(const unsigned short *M, int ld, int k0, int n0) {
-  const int l = threadIdx.x & 63;
-  const int n = n0 + (l & 15), k = k0 + 4 * (l >> 4);
-  bf16x4 v;
-  v[0] = (short)M[(k + 0) * ld + n];
-  v[1] = (short)M[(k + 1) * ld + n];
-  v[2] = (short)M[(k + 2) * ld + n];
-  v[3] = (short)M[(k + 3) * ld + n];
-  return v;
-}
+constexpr int kTilesHid = kHid / 16, kTilesIn = kInPad / 16;
 
-// B operand of a transposed matrix: B[k][n] = M[n][k]
-__device__ __forceinline__ bf16x4 ld_bt(const unsigned short *M, int ld, int k0, int n0) {
-  const int l = threadIdx.x & 63;
-  const unsigned short *p = M + (n0 + (l & 15)) * ld + k0 + 4 * (l >> 4);
-  bf16x4 v;
-  v[0] = (short)p[0];
-  v[1] = (short)p[1];
-  v[2] = (short)p[2];
-  v[3] = (short)p[3];
-  return v;
-}
-
-struct WaveLds {
-  unsigned short xb[16 * kInPad];
-  unsigned short h1b[16 * kHid], h2b[16 * kHid], dzb[16 * kHid], dyb[16 * kOutPad];
-};
-
-// FP32 hidden activations of a tile in the result layout: h[nt][j] is
-// row 4q + j, column 16 nt + r of the layer
+// activations of a tile: FP32 and the BF16 operands the products read
 struct Hidden {
-  floatx4 h1[kHid / 16], h2[kHid / 16];
+  bf16x4 x[kTilesIn], b1[kTilesHid], b2[kTilesHid];
+  floatx4 h1[kTilesHid], h2[kTilesHid];
 };
 
-struct BlockLds {
-  unsigned short w1[kInPad * kHid], w2[kHid * kHid], w3[kHid * kOutPad];
-  float b1[kHid], b2[kHid], b3[kOutPad];
-  WaveLds wave[kBlk / 64];
-};
-
-__device__ void stage_weights(BlockLds &s, const NetDev &net) {
-  for (int i = threadIdx.x; i < kInPad * kHid; i += kBlk) s.w1[i] = net.w1b[i];
-  for (int i = threadIdx.x; i < kHid * kHid; i += kBlk) s.w2[i] = net.w2b[i];
-  for (int i = threadIdx.x; i < kHid * kOutPad; i += kBlk) s.w3[i] = net.w3b[i];
-  for (int i = threadIdx.x; i < kHid; i += kBlk) {
-    s.b1[i] = net.b1[i];
-    s.b2[i] = net.b2[i];
-  }
-  for (int i = threadIdx.x; i < kOutPad; i += kBlk) s.b3[i] = net.b3[i];
-}
-
-// forward pass of one 16-sample tile; rows >= nvalid are zero inputs.
-// Leaves the activations in w; returns this lane's outputs D[4q + j][r].
-__device__ floatx4 forward_tile(const BlockLds &s, WaveLds &w, const float *X, const int64_t *rows,
-                                int nvalid, Hidden &hid) {
-  const int l = threadIdx.x & 63, r = l & 15, q = l >> 4;
-  // inputs -> bf16, zero padded to kInPad columns
-  for (int e = l; e < 16 * kInPad; e += 64) {
-    const int row = e / kInPad, col = e % kInPad;
-    float v = 0.f;
-    if (row < nvalid && col < kIn) v = X[rows[row] * kIn + col];
-    w.xb[e] = to_bf16(v);
-  }
-  __syncthreads();
-  // layer 1
-  for (int nt = 0; nt < kHid / 16; nt++) {
-    floatx4 acc = {0.f, 0.f, 0.f, 0.f};
-    for (int ks = 0; ks < kInPad / 16; ks++) acc = mfma(ld_a(w.xb, kInPad, 0, ks * 16), ld_b(s.w1, kHid, ks * 16, nt * 16), acc);
+// forward pass of one 16-sample tile; row: this lane's sample (r), valid or a
+// zero input. Returns output 4q + j of sample r.
+__device__ __forceinline__ floatx4 forward_tile(const NetDev &net, const float *X, int64_t row, bool valid,
+                                                Hidden &hid) {
+  const int q = (threadIdx.x & 63) >> 4;
+  for (int ks = 0; ks < kTilesIn; ks++) {
+    floatx4 v = {0.f, 0.f, 0.f, 0.f};
     for (int j = 0; j < 4; j++) {
-      const int row = 4 * q + j, col = nt * 16 + r;
-      const float h = tanhf(acc[j] + s.b1[col]);
-      hid.h1[nt][j] = h;
-      w.h1b[row * kHid + col] = to_bf16(h);
+      const int k = 16 * ks + 4 * q + j;
+      if (valid && k < kIn) v[j] = X[row * kIn + k];
     }
+    hid.x[ks] = pack4(v);
   }
-  __syncthreads();
-  // layer 2
-  for (int nt = 0; nt < kHid / 16; nt++) {
+#pragma unroll
+  for (int nt = 0; nt < kTilesHid; nt++) {
     floatx4 acc = {0.f, 0.f, 0.f, 0.f};
-    for (int ks = 0; ks < kHid / 16; ks++) acc = mfma(ld_a(w.h1b, kHid, 0, ks * 16), ld_b(s.w2, kHid, ks * 16, nt * 16), acc);
-    for (int j = 0; j < 4; j++) {
-      const int row = 4 * q + j, col = nt * 16 + r;
-      const float h = tanhf(acc[j] + s.b2[col]);
-      hid.h2[nt][j] = h;
-      w.h2b[row * kHid + col] = to_bf16(h);
-    }
+    for (int ks = 0; ks < kTilesIn; ks++) acc = mfma(ld_w(net.w1f, nt * kTilesIn + ks), hid.x[ks], acc);
+    const float *b = net.b1 + 16 * nt + 4 * q;
+    for (int j = 0; j < 4; j++) hid.h1[nt][j] = tanhf(acc[j] + b[j]);
+    hid.b1[nt] = pack4(hid.h1[nt]);
   }
-  __syncthreads();
-  // layer 3 (linear)
+#pragma unroll
+  for (int nt = 0; nt < kTilesHid; nt++) {
+    floatx4 acc = {0.f, 0.f, 0.f, 0.f};
+    for (int ks = 0; ks < kTilesHid; ks++) acc = mfma(ld_w(net.w2f, nt * kTilesHid + ks), hid.b1[ks], acc);
+    const float *b = net.b2 + 16 * nt + 4 * q;
+    for (int j = 0; j < 4; j++) hid.h2[nt][j] = tanhf(acc[j] + b[j]);
+    hid.b2[nt] = pack4(hid.h2[nt]);
+  }
   floatx4 y = {0.f, 0.f, 0.f, 0.f};
-  for (int ks = 0; ks < kHid / 16; ks++) y = mfma(ld_a(w.h2b, kHid, 0, ks * 16), ld_b(s.w3, kOutPad, ks * 16, 0), y);
-  for (int j = 0; j < 4; j++) y[j] += s.b3[r];
+  for (int ks = 0; ks < kTilesHid; ks++) y = mfma(ld_w(net.w3f, ks), hid.b2[ks], y);
+  for (int j = 0; j < 4; j++) y[j] += net.b3[4 * q + j];
   return y;
 }
 
 __global__ __launch_bounds__(kBlk) void k_mlp_forward(NetDev net, const float *X, int64_t n, float *Y) {
-  __shared__ BlockLds s;
-  stage_weights(s, net);
-  __syncthreads();
-  const int wv = threadIdx.x >> 6, l = threadIdx.x & 63, r = l & 15, q = l >> 4;
-  const int64_t t0 = ((int64_t)blockIdx.x * (kBlk / 64) + wv) * 16;
-  int64_t rows[16];
-  for (int i = 0; i < 16; i++) rows[i] = t0 + i;
-  const int nvalid = (int)(n - t0 < 0 ? 0 : (n - t0 > 16 ? 16 : n - t0));
+  const int l = threadIdx.x & 63, r = l & 15, q = l >> 4;
+  const int64_t row = ((int64_t)blockIdx.x * (kBlk / 64) + (threadIdx.x >> 6)) * 16 + r;
   Hidden hid;
-  const floatx4 y = forward_tile(s, s.wave[wv], X, rows, nvalid, hid);
-  if (r < kOut)
-    for (int j = 0; j < 4; j++) {
-      const int row = 4 * q + j;
-      if (row < nvalid) Y[(t0 + row) * kOut + r] = y[j];
-    }
+  const floatx4 y = forward_tile(net, X, row, row < n, hid);
+  if (q == 0 && row < n)
+    for (int j = 0; j < kOut; j++) Y[row * kOut + j] = y[j];
 }
 
-// one gradient pass: every wavefront takes one 16-sample tile of the batch
-// (sample k of the batch is rows idx[k]), runs forward and backward with the
-// products on matrix cores, and the block writes the sum of its tiles'
-// parameter gradients to part[block][] (wavefronts added in a fixed order, so
-// the result does not depend on timing). Loss = mean over the batch of
-// |y - t|^2; BF16 copies feed every product: inputs, weights, hidden
-// activations, and the output and hidden-layer deltas.
-__device__ __forceinline__ float sum_over_q(float v) {
-  v += __shfl_xor(v, 16, 64);
-  v += __shfl_xor(v, 32, 64);
+// sample k of a batch
+__device__ __forceinline__ int64_t picked_row(const RowPick &p, int64_t k) {
+  if (p.n <= 0) return k;
+  uint64_t z = p.seed + 0x9e3779b97f4a7c15ull * (uint64_t)(k + 1);  // splitmix64
+  z = (z ^ (z >> 30)) * 0xbf58476d1ce4e5b9ull;
+  z = (z ^ (z >> 27)) * 0x94d049bb133111ebull;
+  z ^= z >> 31;
+  return (int64_t)(z % (uint64_t)p.n);
+}
+
+// A tile's operands of the weight-gradient products, sample by sample: rows
+// padded by 8 bytes so that the 16 lanes of a write fall in different banks.
+constexpr int kActStride = kHid + 4, kXStride = kInPad + 4, kYStride = kOutPad + 4;
+struct WaveLds {
+  unsigned short x[16 * kXStride], h1[16 * kActStride], h2[16 * kActStride], d1[16 * kActStride],
+      d2[16 * kActStride], dy[16 * kYStride];
+};
+struct GradLds {
+  WaveLds wave[kBlk / 64];
+  float part[kBlk / 64][kNumParams];  // each wavefront's parameter gradients
+  float loss[kBlk / 64];
+};
+
+// features 16t + 4q .. + 3 of sample r
+__device__ __forceinline__ void put_act(unsigned short *m, int stride, int t, bf16x4 v) {
+  const int l = threadIdx.x & 63;
+  *(bf16x4 *)(m + (l & 15) * stride + 16 * t + 4 * (l >> 4)) = v;
+}
+
+// feature 16t + r of samples 4q .. + 3: the A operand (rows features) and the B
+// operand (columns features) of a product over the samples
+__device__ __forceinline__ bf16x4 get_act(const unsigned short *m, int stride, int t) {
+  const int l = threadIdx.x & 63;
+  const unsigned short *p = m + 4 * (l >> 4) * stride + 16 * t + (l & 15);
+  bf16x4 v;
+  for (int j = 0; j < 4; j++) v[j] = (short)p[j * stride];
   return v;
 }
 
-__global__ __launch_bounds__(kBlk) void k_mlp_grad(NetDev net, const float *X, const float *T,
-                                                    const int64_t *idx, int64_t batch, float *part,
-                                                    float *loss_part) {
-  __shared__ BlockLds s;
-  __shared__ float red[kNumParams];
-  __shared__ float lred[kBlk / 64];
-  stage_weights(s, net);
-  for (int i = threadIdx.x; i < kNumParams; i += kBlk) red[i] = 0.f;
-  __syncthreads();
+// sum over the row of 16 lanes (the tile's samples), by DPP rotations
+__device__ __forceinline__ float row_sum(float v) {
+  v += __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0x128, 0xf, 0xf, true));
+  v += __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0x124, 0xf, 0xf, true));
+  v += __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0x122, 0xf, 0xf, true));
+  v += __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0x121, 0xf, 0xf, true));
+  return v;
+}
+
+// one gradient pass: every wavefront takes one 16-sample tile of the batch,
+// runs forward and backward with the products on matrix cores, and the block
+// writes the sum of its four tiles' parameter gradients to part[block][] (in a
+// fixed order, so the result does not depend on timing). Loss = mean over the
+// batch of |y - t|^2; BF16 copies feed every product: inputs, weights, hidden
+// activations, and the output and hidden-layer deltas. Bound by the latency of
+// one tile's chain (32 tanh a lane, 80 products): 8,192 samples in 21 us on
+// half the chip's CUs; with the weights staged in LDS two bytes at a time and
+// the activations passed through it 30 us.
+__global__ __launch_bounds__(kBlk) void k_mlp_grad(NetDev net, const float *X, const float *T, RowPick pick,
+                                                    int64_t batch, float *part, float *loss_part) {
+  __shared__ GradLds s;
   const int wv = threadIdx.x >> 6, l = threadIdx.x & 63, r = l & 15, q = l >> 4;
   WaveLds &w = s.wave[wv];
-  const int64_t t0 = ((int64_t)blockIdx.x * (kBlk / 64) + wv) * 16;
-  const int nvalid = (int)(batch - t0 < 0 ? 0 : (batch - t0 > 16 ? 16 : batch - t0));
-  int64_t rows[16];
-  for (int i = 0; i < 16; i++) rows[i] = i < nvalid ? (idx ? idx[t0 + i] : t0 + i) : 0;
+  float *out = s.part[wv];
+  const int64_t k = ((int64_t)blockIdx.x * (kBlk / 64) + wv) * 16 + r;
+  const bool valid = k < batch;
+  const int64_t row = valid ? picked_row(pick, k) : 0;
   Hidden hid;
-  const floatx4 y = forward_tile(s, w, X, rows, nvalid, hid);
+  const floatx4 y = forward_tile(net, X, row, valid, hid);
   const float scale = 2.0f / (float)batch;
-  float lsum = 0.f, db3 = 0.f;
-  for (int j = 0; j < 4; j++) {
-    const int row = 4 * q + j;
-    float d = 0.f;
-    if (row < nvalid && r < kOut) {
-      const float e = y[j] - T[rows[row] * kOut + r];
+  float lsum = 0.f;
+  floatx4 d = {0.f, 0.f, 0.f, 0.f};
+  if (valid && q == 0)
+    for (int j = 0; j < kOut; j++) {
+      const float e = y[j] - T[row * kOut + j];
       lsum += e * e;
-      d = scale * e;
+      d[j] = scale * e;
     }
-    db3 += d;
-    w.dyb[row * kOutPad + r] = to_bf16(d);
+  const bf16x4 dyb = pack4(d);
+  for (int t = 0; t < kTilesIn; t++) put_act(w.x, kXStride, t, hid.x[t]);
+  for (int t = 0; t < kTilesHid; t++) {
+    put_act(w.h1, kActStride, t, hid.b1[t]);
+    put_act(w.h2, kActStride, t, hid.b2[t]);
   }
-  __syncthreads();
-  // dW3 = H2^T dY (kHid x kOut)
-  floatx4 gw3[kHid / 16];
-  for (int mt = 0; mt < kHid / 16; mt++) {
-    const floatx4 z = {0.f, 0.f, 0.f, 0.f};
-    gw3[mt] = mfma(ld_at(w.h2b, kHid, mt * 16, 0), ld_b(w.dyb, kOutPad, 0, 0), z);
-  }
-  // dZ2 = (dY W3^T) * (1 - h2^2)
-  float db2[kHid / 16];
-  for (int nt = 0; nt < kHid / 16; nt++) {
-    floatx4 acc = {0.f, 0.f, 0.f, 0.f};
-    acc = mfma(ld_a(w.dyb, kOutPad, 0, 0), ld_bt(s.w3, kOutPad, 0, nt * 16), acc);
-    db2[nt] = 0.f;
+  put_act(w.dy, kYStride, 0, dyb);
+  const floatx4 zero = {0.f, 0.f, 0.f, 0.f};
+  // dZ2 = (dY W3^T) * (1 - h2^2), dZ1 = (dZ2 W2^T) * (1 - h1^2), transposed
+  bf16x4 d2b[kTilesHid];
+#pragma unroll
+  for (int t = 0; t < kTilesHid; t++) {
+    floatx4 v = mfma(ld_w(net.w3t, t), dyb, zero);
+    for (int j = 0; j < 4; j++) v[j] *= 1.0f - hid.h2[t][j] * hid.h2[t][j];
+    d2b[t] = pack4(v);
+    put_act(w.d2, kActStride, t, d2b[t]);
     for (int j = 0; j < 4; j++) {
-      const int row = 4 * q + j, col = nt * 16 + r;
-      const float h = hid.h2[nt][j];
-      const float dz = acc[j] * (1.0f - h * h);
-      db2[nt] += dz;
-      w.dzb[row * kHid + col] = to_bf16(dz);
+      const float b = row_sum(v[j]);
+      if (r == 0) out[kOffB2 + 16 * t + 4 * q + j] = b;
     }
   }
-  __syncthreads();
-  // dW2 = H1^T dZ2 (kHid x kHid)
-  floatx4 gw2[kHid / 16][kHid / 16];
-  for (int mt = 0; mt < kHid / 16; mt++)
-    for (int nt = 0; nt < kHid / 16; nt++) {
-      const floatx4 z = {0.f, 0.f, 0.f, 0.f};
-      gw2[mt][nt] = mfma(ld_at(w.h1b, kHid, mt * 16, 0), ld_b(w.dzb, kHid, 0, nt * 16), z);
-    }
-  // dH1 = dZ2 W2^T
-  floatx4 dh1[kHid / 16];
-  for (int nt = 0; nt < kHid / 16; nt++) {
-    floatx4 acc = {0.f, 0.f, 0.f, 0.f};
-    for (int ks = 0; ks < kHid / 16; ks++)
-      acc = mfma(ld_a(w.dzb, kHid, 0, ks * 16), ld_bt(s.w2, kHid, ks * 16, nt * 16), acc);
-    dh1[nt] = acc;
-  }
-  __syncthreads();  // every read of dZ2 is done
-  float db1[kHid / 16];
-  for (int nt = 0; nt < kHid / 16; nt++) {
-    db1[nt] = 0.f;
+#pragma unroll
+  for (int t = 0; t < kTilesHid; t++) {
+    floatx4 v = zero;
+    for (int ks = 0; ks < kTilesHid; ks++) v = mfma(ld_w(net.w2t, t * kTilesHid + ks), d2b[ks], v);
+    for (int j = 0; j < 4; j++) v[j] *= 1.0f - hid.h1[t][j] * hid.h1[t][j];
+    put_act(w.d1, kActStride, t, pack4(v));
     for (int j = 0; j < 4; j++) {
-      const int row = 4 * q + j, col = nt * 16 + r;
-      const float h = hid.h1[nt][j];
-      const float dz = dh1[nt][j] * (1.0f - h * h);
-      db1[nt] += dz;
-      w.dzb[row * kHid + col] = to_bf16(dz);
+      const float b = row_sum(v[j]);
+      if (r == 0) out[kOffB1 + 16 * t + 4 * q + j] = b;
     }
   }
-  __syncthreads();
-  // dW1 = X^T dZ1 (kInPad x kHid; rows >= kIn are padding)
-  floatx4 gw1[kInPad / 16][kHid / 16];
-  for (int mt = 0; mt < kInPad / 16; mt++)
-    for (int nt = 0; nt < kHid / 16; nt++) {
-      const floatx4 z = {0.f, 0.f, 0.f, 0.f};
-      gw1[mt][nt] = mfma(ld_at(w.xb, kInPad, mt * 16, 0), ld_b(w.dzb, kHid, 0, nt * 16), z);
-    }
-  // bias sums over the tile's rows (lanes r, r+16, r+32, r+48)
-  db3 = sum_over_q(db3);
-  for (int nt = 0; nt < kHid / 16; nt++) {
-    db2[nt] = sum_over_q(db2[nt]);
-    db1[nt] = sum_over_q(db1[nt]);
+  for (int j = 0; j < 4; j++) {
+    const float b = row_sum(d[j]);
+    if (l == 0 && j < kOut) out[kOffB3 + j] = b;
   }
-  for (int off = 32; off > 0; off >>= 1) lsum += __shfl_xor(lsum, off, 64);
-  // the wavefronts add into the block sum one after the other
-  for (int p = 0; p < kBlk / 64; p++) {
-    if (wv == p) {
-      for (int mt = 0; mt < kHid / 16; mt++)
-        if (r < kOut)
-          for (int j = 0; j < 4; j++) red[kOffW3 + (mt * 16 + 4 * q + j) * kOut + r] += gw3[mt][j];
-      for (int mt = 0; mt < kHid / 16; mt++)
-        for (int nt = 0; nt < kHid / 16; nt++)
-          for (int j = 0; j < 4; j++) red[kOffW2 + (mt * 16 + 4 * q + j) * kHid + nt * 16 + r] += gw2[mt][nt][j];
-      for (int mt = 0; mt < kInPad / 16; mt++)
-        for (int nt = 0; nt < kHid / 16; nt++)
-          for (int j = 0; j < 4; j++) {
-            const int m = mt * 16 + 4 * q + j;
-            if (m < kIn) red[kOffW1 + m * kHid + nt * 16 + r] += gw1[mt][nt][j];
-          }
-      if (q == 0) {
-        if (r < kOut) red[kOffB3 + r] += db3;
-        for (int nt = 0; nt < kHid / 16; nt++) {
-          red[kOffB2 + nt * 16 + r] += db2[nt];
-          red[kOffB1 + nt * 16 + r] += db1[nt];
-        }
+  lsum = row_sum(lsum);
+  if (l == 0) s.loss[wv] = lsum;
+  __syncthreads();  // the tile's operands are in LDS
+  // dW3 = H2^T dY, dW2 = H1^T dZ2, dW1 = X^T dZ1 (rows >= kIn are padding)
+  {
+    const bf16x4 b = get_act(w.dy, kYStride, 0);
+    for (int mt = 0; mt < kTilesHid; mt++) {
+      const floatx4 g = mfma(get_act(w.h2, kActStride, mt), b, zero);
+      if (r < kOut)
+        for (int j = 0; j < 4; j++) out[kOffW3 + (mt * 16 + 4 * q + j) * kOut + r] = g[j];
+    }
+  }
+#pragma unroll
+  for (int nt = 0; nt < kTilesHid; nt++) {
+    const bf16x4 b2 = get_act(w.d2, kActStride, nt), b1 = get_act(w.d1, kActStride, nt);
+    for (int mt = 0; mt < kTilesHid; mt++) {
+      const floatx4 g = mfma(get_act(w.h1, kActStride, mt), b2, zero);
+      for (int j = 0; j < 4; j++) out[kOffW2 + (mt * 16 + 4 * q + j) * kHid + nt * 16 + r] = g[j];
+    }
+    for (int mt = 0; mt < kTilesIn; mt++) {
+      const floatx4 g = mfma(get_act(w.x, kXStride, mt), b1, zero);
+      for (int j = 0; j < 4; j++) {
+        const int m = mt * 16 + 4 * q + j;
+        if (m < kIn) out[kOffW1 + m * kHid + nt * 16 + r] = g[j];
       }
-      if (l == 0) lred[wv] = lsum;
     }
-    __syncthreads();
   }
-  for (int i = threadIdx.x; i < kNumParams; i += kBlk) part[(int64_t)blockIdx.x * kNumParams + i] = red[i];
+  __syncthreads();
+  for (int i = threadIdx.x; i < kNumParams; i += kBlk) {
+    float v = 0.f;
+    for (int p = 0; p < kBlk / 64; p++) v += s.part[p][i];
+    part[(int64_t)blockIdx.x * kNumParams + i] = v;
+  }
   if (threadIdx.x == 0) {
     float v = 0.f;
-    for (int k = 0; k < kBlk / 64; k++) v += lred[k];
+    for (int p = 0; p < kBlk / 64; p++) v += s.loss[p];
     loss_part[blockIdx.x] = v;
   }
 }
 
 // sums the blocks' gradient partials (fixed order: deterministic), then one
-// Adam step on the FP32 master parameters and a refresh of the BF16 / padded
-// copies the matrix cores read. adam = 0: only the summed gradient is written.
-__global__ __launch_bounds__(kBlk) void k_mlp_adam(NetDev net, const float *part, int nparts, float *grad,
-                                                   AdamArgs ad) {
-  const int i = blockIdx.x * kBlk + threadIdx.x;
-  if (i == 0 && ad.loss_out) {  // the batch loss of this step
-    float v = 0.f;
-    for (int b = 0; b < nparts; b++) v += ad.loss_part[b];
-    *ad.loss_out = v / (float)ad.batch;
+// Adam step on the FP32 master parameters and a refresh of the copies the
+// matrix cores read. adam = 0: only the summed gradient is written. 64
+// parameters a block, each summed by 16 threads: one thread a parameter, which
+// leaves 22 blocks with 128 loads in a row each, took 34 us of a step, this
+// takes 5. The last block sums the batch loss.
+constexpr int kAdamParams = 64, kAdamSlices = 16;
+__global__ __launch_bounds__(kAdamParams * kAdamSlices) void k_mlp_adam(NetDev net, const float *part, int nparts,
+                                                                        float *grad, AdamArgs ad) {
+  __shared__ float sum[kAdamSlices][kAdamParams];
+  const int c = threadIdx.x % kAdamParams, sl = threadIdx.x / kAdamParams;
+  const bool loss = blockIdx.x == gridDim.x - 1;
+  const int i = blockIdx.x * kAdamParams + c;
+  float v = 0.f;
+  if (loss) {
+    for (int b = threadIdx.x; b < nparts; b += kAdamParams * kAdamSlices) v += ad.loss_part[b];
+  } else if (i < kNumParams) {
+#pragma unroll 8
+    for (int b = sl; b < nparts; b += kAdamSlices) v += part[(int64_t)b * kNumParams + i];
+  }
+  sum[sl][c] = v;
+  __syncthreads();
+  if (sl != 0) return;
+  float gsum = 0.f;
+  for (int k = 0; k < kAdamSlices; k++) gsum += sum[k][c];
+  if (loss) {
+    for (int off = 32; off > 0; off >>= 1) gsum += __shfl_xor(gsum, off, 64);
+    if (c == 0 && ad.loss_out) *ad.loss_out = gsum / (float)ad.batch;
+    return;
   }
   if (i >= kNumParams) return;
-  float gsum = 0.f;
-  for (int b = 0; b < nparts; b++) gsum += part[(int64_t)b * kNumParams + i];
   grad[i] = gsum;
   if (!ad.apply) return;
-  float m = ad.beta1 * net.m[i] + (1.0f - ad.beta1) * gsum;
-  float v = ad.beta2 * net.v[i] + (1.0f - ad.beta2) * gsum * gsum;
+  const float m = ad.beta1 * net.m[i] + (1.0f - ad.beta1) * gsum;
+  const float v2 = ad.beta2 * net.v[i] + (1.0f - ad.beta2) * gsum * gsum;
   net.m[i] = m;
-  net.v[i] = v;
-  const float mh = m / ad.bc1, vh = v / ad.bc2;
+  net.v[i] = v2;
+  const float mh = m / ad.bc1, vh = v2 / ad.bc2;
   const float p = net.params[i] - ad.lr * mh / (sqrtf(vh) + ad.eps);
   net.params[i] = p;
   write_packed(net, i, p);
@@ -594,17 +551,6 @@ __global__ __launch_bounds__(kBlk) void k_mlp_adam(NetDev net, const float *part
 __global__ __launch_bounds__(kBlk) void k_mlp_pack(NetDev net) {
   const int i = blockIdx.x * kBlk + threadIdx.x;
   if (i < kNumParams) write_packed(net, i, net.params[i]);
-}
-
-// batch rows for a training step: uniform with replacement from [0, n)
-__global__ __launch_bounds__(kBlk) void k_sample(int64_t *idx, int64_t batch, int64_t n, uint64_t seed) {
-  const int64_t k = (int64_t)blockIdx.x * kBlk + threadIdx.x;
-  if (k >= batch) return;
-  uint64_t z = seed + 0x9e3779b97f4a7c15ull * (uint64_t)(k + 1);  // splitmix64
-  z = (z ^ (z >> 30)) * 0xbf58476d1ce4e5b9ull;
-  z = (z ^ (z >> 27)) * 0x94d049bb133111ebull;
-  z ^= z >> 31;
-  idx[k] = (int64_t)(z % (uint64_t)n);
 }
 
 // ---------------------------------------------------------------------------
@@ -692,23 +638,18 @@ hipError_t grad_scratch(int device, float **part, float **loss_part) {
   return hipSuccess;
 }
 
-hipError_t launch_mlp_grad(const NetDev &net, const float *X, const float *T, const int64_t *idx,
+hipError_t launch_mlp_grad(const NetDev &net, const float *X, const float *T, const RowPick &pick,
                            int64_t batch, float *part, float *loss_part, hipStream_t s) {
   if (batch <= 0) return hipSuccess;
-  hipLaunchKernelGGL(k_mlp_grad, dim3(grad_blocks(batch)), dim3(kBlk), 0, s, net, X, T, idx, batch, part,
+  hipLaunchKernelGGL(k_mlp_grad, dim3(grad_blocks(batch)), dim3(kBlk), 0, s, net, X, T, pick, batch, part,
                      loss_part);
   return hipGetLastError();
 }
 
 hipError_t launch_mlp_adam(const NetDev &net, const float *part, int nparts, float *grad, const AdamArgs &ad,
                            hipStream_t s) {
-  hipLaunchKernelGGL(k_mlp_adam, dim3(nblk(kNumParams, kBlk)), dim3(kBlk), 0, s, net, part, nparts, grad, ad);
-  return hipGetLastError();
-}
-
-hipError_t launch_sample(int64_t *idx, int64_t batch, int64_t n, uint64_t seed, hipStream_t s) {
-  if (batch <= 0) return hipSuccess;
-  hipLaunchKernelGGL(k_sample, dim3(nblk(batch, kBlk)), dim3(kBlk), 0, s, idx, batch, n, seed);
+  hipLaunchKernelGGL(k_mlp_adam, dim3(nblk(kNumParams, kAdamParams) + 1), dim3(kAdamParams * kAdamSlices), 0, s, net,
+                     part, nparts, grad, ad);
   return hipGetLastError();
 }
 

@@ -36,9 +36,8 @@ struct dem_sq_handle {
   std::vector<void *> net_allocs;
   sqk::NetDev net{};
   float *grad = nullptr, *part = nullptr, *loss_part = nullptr, *loss_hist = nullptr;
-  int64_t *idx = nullptr;
   int part_cap = 0;
-  int64_t idx_cap = 0, loss_cap = 0;
+  int64_t loss_cap = 0;
   int64_t adam_t = 0;
   bool net_ready = false;
   // this device's copy of the allocation-free gradient's workspace
@@ -82,7 +81,7 @@ int ensure_net(dem_sq_handle *h) {
   return DEM_OK;
 }
 
-// batch workspace: gradient partials, loss partials and row indices
+// batch workspace: gradient and loss partials
 int ensure_batch(dem_sq_handle *h, int64_t batch) {
   const int nb = sqk::grad_blocks(batch);
   int rc;
@@ -91,10 +90,6 @@ int ensure_batch(dem_sq_handle *h, int64_t batch) {
       return rc;
     if ((rc = alloc(h, h->net_allocs, (void **)&h->loss_part, sizeof(float) * (size_t)nb))) return rc;
     h->part_cap = nb;
-  }
-  if (batch > h->idx_cap) {
-    if ((rc = alloc(h, h->net_allocs, (void **)&h->idx, sizeof(int64_t) * (size_t)batch))) return rc;
-    h->idx_cap = batch;
   }
   return DEM_OK;
 }
@@ -353,8 +348,9 @@ int dem_sq_net_init(dem_sq_handle *h, uint64_t seed) {
     sqk::NetDev &n = h->net;
     if ((rc = A((void **)&n.params, sizeof(float) * sqk::kNumParams)) || (rc = A((void **)&n.m, sizeof(float) * sqk::kNumParams)) ||
         (rc = A((void **)&n.v, sizeof(float) * sqk::kNumParams)) ||
-        (rc = A((void **)&n.w1b, 2 * sqk::kInPad * sqk::kHid)) || (rc = A((void **)&n.w2b, 2 * sqk::kHid * sqk::kHid)) ||
-        (rc = A((void **)&n.w3b, 2 * sqk::kHid * sqk::kOutPad)) || (rc = A((void **)&n.b1, sizeof(float) * sqk::kHid)) ||
+        (rc = A((void **)&n.w1f, 2 * sqk::kInPad * sqk::kHid)) || (rc = A((void **)&n.w2f, 2 * sqk::kHid * sqk::kHid)) ||
+        (rc = A((void **)&n.w3f, 2 * sqk::kHid * sqk::kOutPad)) || (rc = A((void **)&n.w2t, 2 * sqk::kHid * sqk::kHid)) ||
+        (rc = A((void **)&n.w3t, 2 * sqk::kHid * sqk::kOutPad)) || (rc = A((void **)&n.b1, sizeof(float) * sqk::kHid)) ||
         (rc = A((void **)&n.b2, sizeof(float) * sqk::kHid)) || (rc = A((void **)&n.b3, sizeof(float) * sqk::kOutPad)) ||
         (rc = A((void **)&h->grad, sizeof(float) * sqk::kNumParams)))
       return rc;
@@ -382,8 +378,9 @@ int dem_sq_net_set_params(dem_sq_handle *h, const float *params) {
   SQCHK(h, hipMemcpy(n.params, params, sizeof(float) * sqk::kNumParams, hipMemcpyHostToDevice));
   SQCHK(h, hipMemset(n.m, 0, sizeof(float) * sqk::kNumParams));
   SQCHK(h, hipMemset(n.v, 0, sizeof(float) * sqk::kNumParams));
-  SQCHK(h, hipMemset(n.w1b, 0, 2 * sqk::kInPad * sqk::kHid));
-  SQCHK(h, hipMemset(n.w3b, 0, 2 * sqk::kHid * sqk::kOutPad));
+  SQCHK(h, hipMemset(n.w1f, 0, 2 * sqk::kInPad * sqk::kHid));
+  SQCHK(h, hipMemset(n.w3f, 0, 2 * sqk::kHid * sqk::kOutPad));
+  SQCHK(h, hipMemset(n.w3t, 0, 2 * sqk::kHid * sqk::kOutPad));
   SQCHK(h, hipMemset(n.b3, 0, sizeof(float) * sqk::kOutPad));
   SQCHK(h, sqk::launch_mlp_pack(n, h->stream));
   SQCHK(h, hipStreamSynchronize(h->stream));
@@ -434,8 +431,6 @@ int dem_sq_net_gradient(dem_sq_handle *h, int64_t n, const float *X, const float
     free_list(tmp);
     return rc;
   }
-  std::vector<int64_t> rows((size_t)n);
-  for (int64_t k = 0; k < n; k++) rows[(size_t)k] = k;
   sqk::AdamArgs ad{};
   ad.apply = 0;
   ad.loss_part = h->loss_part;
@@ -443,8 +438,7 @@ int dem_sq_net_gradient(dem_sq_handle *h, int64_t n, const float *X, const float
   ad.batch = n;
   hipError_t e = hipMemcpy(dX, X, sizeof(float) * sqk::kIn * n, hipMemcpyHostToDevice);
   if (e == hipSuccess) e = hipMemcpy(dT, T, sizeof(float) * sqk::kOut * n, hipMemcpyHostToDevice);
-  if (e == hipSuccess) e = hipMemcpy(h->idx, rows.data(), sizeof(int64_t) * n, hipMemcpyHostToDevice);
-  if (e == hipSuccess) e = sqk::launch_mlp_grad(h->net, dX, dT, h->idx, n, h->part, h->loss_part, h->stream);
+  if (e == hipSuccess) e = sqk::launch_mlp_grad(h->net, dX, dT, sqk::RowPick{}, n, h->part, h->loss_part, h->stream);
   if (e == hipSuccess) e = sqk::launch_mlp_adam(h->net, h->part, sqk::grad_blocks(n), h->grad, ad, h->stream);
   if (e == hipSuccess) e = hipStreamSynchronize(h->stream);
   if (e == hipSuccess) e = hipMemcpy(grad, h->grad, sizeof(float) * sqk::kNumParams, hipMemcpyDeviceToHost);
@@ -475,7 +469,7 @@ int dem_sq_net_gradient_noalloc(dem_sq_handle *h, int64_t n, const float *X, con
   ad.loss_part = h->scr_loss;
   ad.loss_out = loss;
   ad.batch = n;
-  SQCHK(h, sqk::launch_mlp_grad(h->net, X, T, nullptr, n, h->scr_part, h->scr_loss, h->stream));
+  SQCHK(h, sqk::launch_mlp_grad(h->net, X, T, sqk::RowPick{}, n, h->scr_part, h->scr_loss, h->stream));
   SQCHK(h, sqk::launch_mlp_adam(h->net, h->scr_part, sqk::grad_blocks(n), grad, ad, h->stream));
   SQCHK(h, hipStreamSynchronize(h->stream));
   return DEM_OK;
@@ -510,8 +504,8 @@ int dem_sq_net_train(dem_sq_handle *h, int64_t steps, int64_t batch, float lr, u
     ad.bc1 = (float)(1.0 - std::pow(0.9, (double)h->adam_t));
     ad.bc2 = (float)(1.0 - std::pow(0.999, (double)h->adam_t));
     ad.loss_out = h->loss_hist + s;
-    SQCHK(h, sqk::launch_sample(h->idx, batch, h->n, seed + 0x632be59bd9b4e019ull * (uint64_t)s, h->stream));
-    SQCHK(h, sqk::launch_mlp_grad(h->net, h->X, h->T, h->idx, batch, h->part, h->loss_part, h->stream));
+    const sqk::RowPick pick{h->n, seed + 0x632be59bd9b4e019ull * (uint64_t)s};
+    SQCHK(h, sqk::launch_mlp_grad(h->net, h->X, h->T, pick, batch, h->part, h->loss_part, h->stream));
     SQCHK(h, sqk::launch_mlp_adam(h->net, h->part, nb, h->grad, ad, h->stream));
   }
   SQCHK(h, hipEventRecord(h->ev[1], h->stream));
