@@ -21,6 +21,19 @@ constexpr uint32_t kCarryBit = 0x40000000u;
 constexpr uint32_t kIndexMask = 0x3fffffffu;
 constexpr int kMetaCountMask = 0xffff;       // meta[i]: low 16 bits = list length
 constexpr int kMetaWallShift = 16;           // bits 16..21: wall history present
+// Bits 22..31 of meta: how far the particle is from where the last build saw
+// it, the common drift taken off, in units of skin / kReachUnits, rounded up
+// (kReachMax: that far or more). Two particles can touch only when the gap
+// the build saw is no more than the sum of their distances, so a step looks at
+// a list entry only if its gap is within the particle's own distance plus the
+// largest one of all (Ctrl::reach).
+constexpr int kMetaDevShift = 22;
+constexpr int kReachUnits = 512, kReachMax = 1023;
+// AuxBuf::lev holds a two-bit gap class for each of a row's first kLevSlots
+// entries (bit s: low, bit 16 + s: high): class c > 0 when the gap is at least
+// kReachGap[c], the largest such c. Entries past those are always looked at.
+constexpr int kLevSlots = 16;
+constexpr int kReachGap[4] = {0, 32, 88, 176};
 constexpr int kMaxMeshes = 4;
 constexpr int kMeshSlots = 8;       // contact-history slots per particle and mesh
 constexpr int kMaxMeshCand = 32;    // candidate triangles per particle (all meshes)
@@ -61,6 +74,8 @@ struct DevParams {
   double triggersq;        // 0.25 * skin * skin (neighbor.cpp:290)
   int neigh_every;         // neigh_modify every (>= 1)
   int neigh_check;         // neigh_modify check yes (1) / no (0)
+  int reach_on;            // rows are walked by reach (check yes and skin > 0)
+  float reach_scale;       // kReachUnits / skin
   double skin, cdf;
   double cdm;              // contactDistanceMultiplier = cdf * cdf (pair_gran_base.h:224)
   int close_band;          // cdf > 1: pairs within cdf * radsum that do not touch
@@ -138,6 +153,10 @@ struct Ctrl {
   // point) the particles exert on each mesh, at the last counted pass
   double mesh_force[kMaxMeshes][6];
   unsigned long long nlost;  // atoms beyond an f face at the last build
+  // since the last build: the largest distance of a particle (kMetaDevShift),
+  // and the drift it is taken from, of steps of even and odd index
+  int reach, pad3;
+  double drift[2][3];
 };
 
 // Particle state read by neighbors: ping-pong buffered across steps.
@@ -152,7 +171,8 @@ struct StateBuf {
 struct AuxBuf {
   int *tag;
   int *orig;      // caller index
-  int *meta;      // list length | wall-history bits
+  int *meta;      // list length | wall-history bits | distance since the build
+  uint32_t *lev;  // gap classes of the row's first entries (kReachGap)
   void *whist;    // wall history, [wall][hist_w][cap], double or float
   int *mslot;     // mesh history slots: triangle index or -1, [mesh][slot][cap]
   void *mhist;    // mesh history, [mesh][slot][hist_w][cap] (shear, then the epsd2 rolling torque)
@@ -234,6 +254,7 @@ struct StepArgs {
   // moving meshes, blocks [pblocks, gridDim) rotate the meshes into the next
   // step's geometry buffer (mv.dst) while the others compute this step
   int variant, pblocks, move_mesh;
+  int drift_from;      // k_initial: the drift slot of the last run's final step
   int step_from_ctrl;  // step = ctrl->step_base + step, ago_next = ctrl->ago_base + step
   MeshMoveArgs mv;
 };

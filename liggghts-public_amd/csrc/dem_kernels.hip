@@ -80,6 +80,62 @@ __device__ __forceinline__ void min_image(const DevParams &p, double xi, double 
 }
 
 
+// the distance field of meta for a displacement of squared length rsq
+__device__ __forceinline__ int dev_units(const DevParams &p, double rsq) {
+  // rounded up past the conversion's and the root's error
+  const float u = sqrtf((float)rsq) * (p.reach_scale * 1.00001f);
+  return u < (float)(kReachMax - 1) ? (int)u + 1 : kReachMax;
+}
+
+// Raises Ctrl::reach to a wavefront's largest distance. In steps of 16 units,
+// so that between two builds a wavefront has at most 64 occasions to touch it.
+__device__ __forceinline__ void raise_reach(Ctrl *ctrl, int dev, int known) {
+  for (int off = 32; off > 0; off >>= 1) {
+    const int o = __shfl_xor(dev, off, 64);
+    dev = o > dev ? o : dev;
+  }
+  const int level = (dev + 15) & ~15;
+  if (level > known && (threadIdx.x & 63) == 0 &&
+      level > __hip_atomic_load(&ctrl->reach, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
+    atomicMax(&ctrl->reach, level);
+}
+
+// which of a row's first kLevSlots entries can touch at this step, as bits
+__device__ __forceinline__ uint32_t row_reach(int meta, uint32_t lev, int reach) {
+  const int q = (int)((uint32_t)meta >> kMetaDevShift) + reach;
+  const uint32_t lo = lev, hi = lev >> 16;
+  return q < kReachGap[1] ? ~(lo | hi) : (q < kReachGap[2] ? ~hi : (q < kReachGap[3] ? ~(lo & hi) : ~0u));
+}
+
+// The list slots a particle's pair phase looks at, in ascending order, GROUP
+// at a time: of the first 32 slots those of `mask`, then every one below cnt.
+struct RowWalk {
+  uint32_t mask;
+  int base, cnt;
+  __device__ __forceinline__ void start(uint32_t first, int n) {
+    base = 0;
+    cnt = n;
+    mask = first & (n < 32 ? (1u << n) - 1u : ~0u);
+    skip();
+  }
+  __device__ __forceinline__ void skip() {
+    while (mask == 0u && base + 32 < cnt) {
+      base += 32;
+      mask = cnt - base < 32 ? (1u << (cnt - base)) - 1u : ~0u;
+    }
+  }
+  __device__ __forceinline__ bool any() const { return mask != 0u; }
+  // the next slots of the current 32 (-1: no more of them)
+  template <int GROUP>
+  __device__ __forceinline__ void take(int (&ks)[GROUP]) {
+#pragma unroll
+    for (int u = 0; u < GROUP; u++) {
+      ks[u] = mask ? base + __builtin_ctz(mask) : -1;
+      mask &= mask - 1u;
+    }
+  }
+};
+
 template <typename T> struct OmgT;
 template <> struct OmgT<double> { typedef double4 type; };
 template <> struct OmgT<float> { typedef float4 type; };
@@ -731,7 +787,7 @@ __device__ __forceinline__ void mesh_move_block(const MeshMoveArgs &a, const int
 }
 
 // The surfacesClose branch of the pair loop (pair_gran_base.h:414-417) for the
-// entries of bit mask `close` (group k0, entries ent): within cdf * radsum but
+// entries of bit mask `close` (list slots ks, entries ent): within cdf * radsum but
 // not touching. ContactModel::surfacesClose zeroes the shear history
 // (tangential_model_history.h:358-369) and the epsd2 rolling torque
 // (rolling_model_epsd2.h:144-151) and leaves the contact flag nonzero only if
@@ -740,7 +796,7 @@ __device__ __forceinline__ void mesh_move_block(const MeshMoveArgs &a, const int
 // from a carry-over at the last build.
 template <typename T, bool GEN, int GROUP>
 __device__ __forceinline__ void close_entries(const StepArgs &a, const Model &pm, const int i,
-                                              const int k0, uint32_t close,
+                                              const int (&ks)[GROUP], uint32_t close,
                                               const uint32_t (&ent)[GROUP], T *hist,
                                               const size_t cap, const size_t hw) {
   const bool keeps = !(GEN && pm.nohist);
@@ -748,8 +804,13 @@ __device__ __forceinline__ void close_entries(const StepArgs &a, const Model &pm
   while (close) {
     const int u = __builtin_ctz(close);
     close &= close - 1u;
-    const int k = k0 + u;
-    const uint32_t e = ent[u];
+    int k = ks[0];
+    uint32_t e = ent[0];
+#pragma unroll
+    for (int v = 1; v < GROUP; v++) {
+      k = u == v ? ks[v] : k;
+      e = u == v ? ent[v] : e;
+    }
     if (keeps) {
       const T z[3] = {T(0), T(0), T(0)};
       const size_t hb = hist_at(k, i, cap, hist_rec((int)hw));
@@ -858,10 +919,10 @@ __device__ __forceinline__ void pair_contact(const StepArgs &a, const Model &pm,
   if (!flagged) a.list.nbr[(size_t)k * cap + i] = e | kFlagBit;
 }
 
-// Broad phase of list entries k0 .. k0+GROUP-1 of particle i (cnt entries):
+// Broad phase of the list entries in slots ks of particle i (-1: none):
 // the index loads of the group are independent, then its position gathers,
 // so a wavefront has GROUP memory requests in flight instead of one
-// dependent chain per entry. Entries past cnt gather particle `pad` (a valid
+// dependent chain per entry. Empty slots gather particle `pad` (a valid
 // index: i itself, or 0 for a lane past the last particle) and are ignored.
 // Returns the touching entries as bits; entries in the surfacesClose band are
 // handled here.
@@ -871,14 +932,14 @@ __device__ __forceinline__ void pair_contact(const StepArgs &a, const Model &pm,
 // loading it here keeps that latency out of the contact law's chain.
 template <typename T, bool GEN, int GROUP>
 __device__ __forceinline__ uint32_t broad_phase(const StepArgs &a, const Model &pm, const int i,
-                                                const int pad, const int cnt, const int k0,
+                                                const int pad, const int (&ks)[GROUP],
                                                 const double4 &pi, uint32_t (&ent)[GROUP],
                                                 T (*hpre)[3] = nullptr) {
   const DevParams &p = a.prm;
   const size_t cap = (size_t)a.cap;
 #pragma unroll
   for (int u = 0; u < GROUP; u++)
-    ent[u] = (k0 + u < cnt) ? a.list.nbr[(size_t)(k0 + u) * cap + i] : (uint32_t)pad;
+    ent[u] = ks[u] >= 0 ? a.list.nbr[(size_t)ks[u] * cap + i] : (uint32_t)pad;
   double4 pj[GROUP];
 #pragma unroll
   for (int u = 0; u < GROUP; u++) pj[u] = a.in.pos[ent[u] & kIndexMask];
@@ -887,7 +948,7 @@ __device__ __forceinline__ uint32_t broad_phase(const StepArgs &a, const Model &
 #pragma unroll
     for (int u = 0; u < GROUP; u++) {
       hpre[u][0] = hpre[u][1] = hpre[u][2] = T(0);
-      if (k0 + u < cnt && (ent[u] & kFlagBit)) load_rec3(hist + hist_at(k0 + u, i, cap, 4), hpre[u]);
+      if (ks[u] >= 0 && (ent[u] & kFlagBit)) load_rec3(hist + hist_at(ks[u], i, cap, 4), hpre[u]);
     }
   }
   double dx[GROUP], dy[GROUP], dz[GROUP];
@@ -909,7 +970,7 @@ __device__ __forceinline__ uint32_t broad_phase(const StepArgs &a, const Model &
   for (int u = 0; u < GROUP; u++) {
     const double rsq = dx[u] * dx[u] + dy[u] * dy[u] + dz[u] * dz[u];
     const double radsum = pi.w + pj[u].w;
-    if (k0 + u < cnt) {
+    if (ks[u] >= 0) {
       if (rsq < radsum * radsum)
         bits |= 1u << u;
       else if (p.close_band && rsq < p.cdm * radsum * radsum)
@@ -918,7 +979,7 @@ __device__ __forceinline__ uint32_t broad_phase(const StepArgs &a, const Model &
   }
   if (close) {
     const size_t hw = GEN ? (size_t)p.hist_w : 3;
-    close_entries<T, GEN, GROUP>(a, pm, i, k0, close, ent, (T *)a.list.hist, cap, hw);
+    close_entries<T, GEN, GROUP>(a, pm, i, ks, close, ent, (T *)a.list.hist, cap, hw);
   }
   return bits;
 }
@@ -953,7 +1014,7 @@ struct WaveLds {
 // the wavefront takes part; lanes past the last particle have cnt = 0.
 template <typename T, bool GEN, int GROUP>
 __device__ __forceinline__ void pair_forces_wave(const StepArgs &a, const Model &pm, const int i,
-                                                 const int pad, const int cnt, const double4 &pi,
+                                                 const int pad, RowWalk walk, const double4 &pi,
                                                  T &fx, T &fy,
                                                  T &fz, T &tx, T &ty, T &tz,
                                                  unsigned long long &my_contacts,
@@ -963,15 +1024,12 @@ __device__ __forceinline__ void pair_forces_wave(const StepArgs &a, const Model 
   const int lane = threadIdx.x & 63;
   const int ibase = i - lane;  // particle of lane 0
   const unsigned long long below = (1ull << lane) - 1ull;
-  int kmax = cnt;
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) {
-    const int o = __shfl_xor(kmax, off, 64);
-    kmax = o > kmax ? o : kmax;
-  }
-  for (int k0 = 0; k0 < kmax; k0 += GROUP) {
+  while (__ballot(walk.any()) != 0ull) {
     uint32_t ent[GROUP];
-    const uint32_t bits = broad_phase<T, GEN, GROUP>(a, pm, i, pad, cnt, k0, pi, ent);
+    int ks[GROUP];
+    walk.take(ks);
+    walk.skip();
+    const uint32_t bits = broad_phase<T, GEN, GROUP>(a, pm, i, pad, ks, pi, ent);
     // queue position of this lane's entry u: the touching entries of slots
     // below u, then those of lower lanes at slot u
     int pos[GROUP];
@@ -984,7 +1042,7 @@ __device__ __forceinline__ void pair_forces_wave(const StepArgs &a, const Model 
     }
 #pragma unroll
     for (int u = 0; u < GROUP; u++)
-      if ((bits >> u) & 1u) L.queue[pos[u]] = make_uint2(ent[u], ((uint32_t)lane << 16) | (uint32_t)(k0 + u));
+      if ((bits >> u) & 1u) L.queue[pos[u]] = make_uint2(ent[u], ((uint32_t)lane << 16) | (uint32_t)ks[u]);
     my_contacts += (unsigned long long)__popc(bits);
     wave_sync();
     for (int c0 = 0; c0 < total; c0 += 64) {
@@ -1066,39 +1124,45 @@ struct PairLdsT<T, GROUP, 2> {
 // are in L.pos / L.vel / L.omg, staged by the caller.
 template <typename T, bool GEN, int GROUP>
 __device__ __forceinline__ void pair_forces_rowq(const StepArgs &a, const Model &pm, const int i,
-                                                 const int pad, const int cnt, T &fx, T &fy,
+                                                 const int pad, RowWalk walk, T &fx, T &fy,
                                                  T &fz, T &tx, T &ty, T &tz,
                                                  unsigned long long &my_contacts, RowLds<T> &L) {
-  static_assert(32 % GROUP == 0, "a round holds whole groups");
   typedef typename OmgT<T>::type omg_t;
   const DevParams &p = a.prm;
   const size_t cap = (size_t)a.cap;
   const int lane = threadIdx.x & 63;
   const int ibase = i - lane;  // particle of lane 0
-  int kmax = cnt;
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) {
-    const int o = __shfl_xor(kmax, off, 64);
-    kmax = o > kmax ? o : kmax;
-  }
-  for (int r0 = 0; r0 < kmax; r0 += 32) {
-    const int rend = kmax < r0 + 32 ? kmax : r0 + 32;
+  // a round is the 32 slots a lane's walk stands at; every lane starts at 0
+  // and moves to its next 32 with the others
+  for (int r0 = 0; __ballot(walk.any()) != 0ull; r0 += 32) {
     uint32_t tmask = 0u;
     int c = 0;
-    for (int k0 = r0; k0 < rend; k0 += GROUP) {
+    while (__ballot(walk.any() && walk.base == r0) != 0ull) {
       uint32_t ent[GROUP];
+      int ks[GROUP];
+      if (walk.base == r0) {
+        walk.take(ks);
+      } else {
+#pragma unroll
+        for (int u = 0; u < GROUP; u++) ks[u] = -1;
+      }
       const double4 pi = L.pos[lane];
-      uint32_t bits = broad_phase<T, GEN, GROUP>(a, pm, i, pad, cnt, k0, pi, ent);
-      tmask |= bits << (k0 - r0);
+      uint32_t bits = broad_phase<T, GEN, GROUP>(a, pm, i, pad, ks, pi, ent);
       while (bits) {
         const int u = __builtin_ctz(bits);
         bits &= bits - 1u;
         uint32_t e = ent[0];
+        int k = ks[0];
 #pragma unroll
-        for (int v = 1; v < GROUP; v++) e = u == v ? ent[v] : e;
+        for (int v = 1; v < GROUP; v++) {
+          e = u == v ? ent[v] : e;
+          k = u == v ? ks[v] : k;
+        }
+        tmask |= 1u << (k - r0);
         if (c < kRowStash) L.stash[c][lane] = e;
         c++;
       }
+      if (walk.base == r0) walk.skip();
     }
     my_contacts += (unsigned long long)c;
     int incl = c;
@@ -1173,7 +1237,8 @@ template <typename T, bool MESH, int GROUP, bool GEN, int WAVE>
 __device__ __forceinline__ void step_particle(const StepArgs &a, const int i, const bool active,
                                               unsigned long long &my_contacts,
                                               unsigned long long &my_wall, int &my_inst,
-                                              bool &displaced, const long long ago_next,
+                                              bool &displaced, int &dev, const int reach,
+                                              const double *drift, const long long ago_next,
                                               typename PairLdsT<T, GROUP, WAVE>::type *lds) {
   typedef typename OmgT<T>::type omg_t;
   const DevParams &p = a.prm;
@@ -1197,38 +1262,45 @@ __device__ __forceinline__ void step_particle(const StepArgs &a, const int i, co
   my_inst = wbits >> kTypeBits;
   const int meta0 = active ? a.aux.meta[i] : 0;
   int meta = meta0;
-  const int cnt = meta & kMetaCountMask;
+  RowWalk walk;
+  {
+    const uint32_t near = (p.reach_on && active) ? row_reach(meta0, a.aux.lev[i], reach) : ~0u;
+    walk.start(near | ~((1u << kLevSlots) - 1u), meta & kMetaCountMask);
+  }
   const T dt = (T)p.dt;
   const Model pm = model_from_bits(p.pair_model);
   T fx = T(0), fy = T(0), fz = T(0), tx = T(0), ty = T(0), tz = T(0);
 
   if (WAVE == 1 || WAVE == 2) {
     if constexpr (WAVE == 2) {
-      pair_forces_rowq<T, GEN, GROUP>(a, pm, i, ii, cnt, fx, fy, fz, tx, ty, tz, my_contacts, *lds);
+      pair_forces_rowq<T, GEN, GROUP>(a, pm, i, ii, walk, fx, fy, fz, tx, ty, tz, my_contacts, *lds);
       const int lane = threadIdx.x & 63;
       pi = lds->pos[lane];
       vi = lds->vel[lane];
       wi = lds->omg[lane];
     } else
-      pair_forces_wave<T, GEN, GROUP>(a, pm, i, ii, cnt, pi, fx, fy, fz, tx, ty, tz, my_contacts, *lds);
+      pair_forces_wave<T, GEN, GROUP>(a, pm, i, ii, walk, pi, fx, fy, fz, tx, ty, tz, my_contacts, *lds);
     if (!active) return;
   } else {
     // Touching entries of a group are resolved one by one, their list
     // entries selected from the group's registers.
-    for (int k0 = 0; k0 < cnt; k0 += GROUP) {
+    for (; walk.any(); walk.skip()) {
       uint32_t ent[GROUP];
+      int ks[GROUP];
+      walk.take(ks);
       constexpr bool PRE = WAVE == 3 && !GEN;
       T hpre[GROUP][3];
-      uint32_t bits = broad_phase<T, GEN, GROUP>(a, pm, i, i, cnt, k0, pi, ent, PRE ? hpre : nullptr);
+      uint32_t bits = broad_phase<T, GEN, GROUP>(a, pm, i, i, ks, pi, ent, PRE ? hpre : nullptr);
       while (bits) {
         const int u = __builtin_ctz(bits);
-        const int k = k0 + u;
         bits &= bits - 1u;
         uint32_t e = ent[0];
+        int k = ks[0];
         T sh[3] = {hpre[0][0], hpre[0][1], hpre[0][2]};
 #pragma unroll
         for (int v = 1; v < GROUP; v++) {
           e = u == v ? ent[v] : e;
+          k = u == v ? ks[v] : k;
           if (PRE)
             for (int d = 0; d < 3; d++) sh[d] = u == v ? hpre[v][d] : sh[d];
         }
@@ -1405,18 +1477,25 @@ __device__ __forceinline__ void step_particle(const StepArgs &a, const int i, co
       wz += dtir * tz;
       // Neighbor::decide (neighbor.cpp:1366-1371) with delay 0, and
       // Neighbor::check_distance (neighbor.cpp:1436-1443)
-      if (ago_next % p.neigh_every == 0) {
-        if (p.neigh_check) {
+      const bool decide = ago_next % p.neigh_every == 0;
+      if (p.neigh_check) {
+        if (decide || p.reach_on) {
           const double hx = x - a.xhold[i];
           const double hy = y - a.xhold[cap + i];
           const double hz = z - a.xhold[2 * cap + i];
           const double rsq = hx * hx + hy * hy + hz * hz;
           // the lane may hold several tiles (persistent grid): keep a
           // request an earlier tile made
-          displaced = displaced || rsq > p.triggersq;
-        } else {
-          displaced = true;
+          displaced = displaced || (decide && rsq > p.triggersq);
+          if (p.reach_on) {
+            const double ex = hx - drift[0], ey = hy - drift[1], ez = hz - drift[2];
+            const int u = dev_units(p, ex * ex + ey * ey + ez * ez);
+            dev = u > dev ? u : dev;
+            meta = (meta & ((1 << kMetaDevShift) - 1)) | (int)((uint32_t)u << kMetaDevShift);
+          }
         }
+      } else if (decide) {
+        displaced = true;
       }
     }
     a.out.pos[i] = make_double4(x, y, z, pi.w);
@@ -1462,6 +1541,21 @@ __global__ __launch_bounds__(BLOCK) void k_step(StepArgs a) {
   Lds *lds = &lds_all[kWaveLds ? (threadIdx.x >> 6) : 0];
   unsigned long long my_contacts = 0, my_wall = 0;
   bool displaced = false;
+  // the drift the particles' distances are taken from: one particle's path
+  // since the build, so that a cloud moving as one keeps its rows' reach. Any
+  // common vector serves; it is advanced by that particle's velocity as it
+  // stands in this launch's input, which every wavefront reads alike.
+  int dev = 0;
+  const int reach = a.ctrl->reach;
+  double drift[3] = {0.0, 0.0, 0.0};
+  if (p.reach_on && a.do_initial) {
+    const double *d0 = a.ctrl->drift[step & 1];
+    const double4 v = a.in.vel[a.n >> 1];
+    drift[0] = d0[0] + p.dt * v.x;
+    drift[1] = d0[1] + p.dt * v.y;
+    drift[2] = d0[2] + p.dt * v.z;
+    if (blockIdx.x == 0 && threadIdx.x < 3) a.ctrl->drift[(step + 1) & 1][threadIdx.x] = drift[threadIdx.x];
+  }
   const int ntiles = (a.n + BLOCK - 1) / BLOCK;
   for (int tile = xcd_block(a.pblocks); tile < ntiles; tile += a.pblocks) {
     const int i = tile * BLOCK + threadIdx.x;
@@ -1469,7 +1563,7 @@ __global__ __launch_bounds__(BLOCK) void k_step(StepArgs a) {
     if (kWaveLds || active) {
       unsigned long long c = 0, w = 0;
       int inst = 0;
-      step_particle<T, MESH, GROUP, GEN, WAVE>(a, i, active, c, w, inst, displaced, ago_next, lds);
+      step_particle<T, MESH, GROUP, GEN, WAVE>(a, i, active, c, w, inst, displaced, dev, reach, drift, ago_next, lds);
       my_contacts += c;
       my_wall += w;
       if (active && a.count && a.inst_stats) {
@@ -1479,6 +1573,7 @@ __global__ __launch_bounds__(BLOCK) void k_step(StepArgs a) {
     }
   }
 
+  if (p.reach_on && a.do_initial) raise_reach(a.ctrl, dev, reach);
   // rebuild request for the next step
   if (__ballot(displaced) != 0ull) {
     if ((threadIdx.x & 63) == 0)
@@ -1794,6 +1889,9 @@ __global__ __launch_bounds__(kBlock) void k_initial(StepArgs a) {
   typedef typename OmgT<T>::type omg_t;
   const int i = blockIdx.x * kBlock + threadIdx.x;
   bool displaced = false;
+  int dev = 0;
+  const int reach = a.ctrl->reach;
+  if (i < 3 && a.drift_from != 1) a.ctrl->drift[1][i] = a.ctrl->drift[a.drift_from][i];  // step 1 reads slot 1
   if (i < a.n) {
     const DevParams &p = a.prm;
     const size_t cap = (size_t)a.cap;
@@ -1813,17 +1911,24 @@ __global__ __launch_bounds__(kBlock) void k_initial(StepArgs a) {
     a.in.pos[i] = make_double4(x, y, z, pi.w);
     a.in.vel[i] = make_double4(vx, vy, vz, vi.w);
     ((omg_t *)a.in.omg)[i] = wi;
-    if (a.ago_next % p.neigh_every == 0) {
-      if (p.neigh_check) {
-        const double hx = x - a.xhold[i];
-        const double hy = y - a.xhold[cap + i];
-        const double hz = z - a.xhold[2 * cap + i];
-        displaced = hx * hx + hy * hy + hz * hz > p.triggersq;
-      } else {
-        displaced = true;
+    const bool decide = a.ago_next % p.neigh_every == 0;
+    if (p.neigh_check) {
+      const double hx = x - a.xhold[i];
+      const double hy = y - a.xhold[cap + i];
+      const double hz = z - a.xhold[2 * cap + i];
+      displaced = decide && hx * hx + hy * hy + hz * hz > p.triggersq;
+      if (p.reach_on) {
+        // the drift stays as the last step left it: the velocities change in place here
+        const double *d0 = a.ctrl->drift[a.drift_from];
+        const double ex = hx - d0[0], ey = hy - d0[1], ez = hz - d0[2];
+        dev = dev_units(p, ex * ex + ey * ey + ez * ez);
+        a.aux.meta[i] = (a.aux.meta[i] & ((1 << kMetaDevShift) - 1)) | (int)((uint32_t)dev << kMetaDevShift);
       }
+    } else {
+      displaced = decide;
     }
   }
+  if (a.prm.reach_on) raise_reach(a.ctrl, dev, reach);
   if (__ballot(displaced) != 0ull && (threadIdx.x & 63) == 0)
     atomicMin((unsigned long long *)&a.ctrl->stop_at, 1ull);
 }
@@ -2009,7 +2114,7 @@ __global__ __launch_bounds__(kBlock) void k_gather(RebuildArgs a) {
   a.aalt.tag[i] = a.acur.tag[o];
   a.aalt.orig[i] = a.acur.orig[o];
   const int meta = a.acur.meta[o];
-  a.aalt.meta[i] = meta & ~kMetaCountMask;
+  a.aalt.meta[i] = meta & ((1 << kMetaDevShift) - 1) & ~kMetaCountMask;  // the wall-history bits
   const T *wi = (const T *)a.acur.whist;
   T *wo = (T *)a.aalt.whist;
   const int hw = a.prm.hist_w;
@@ -2044,6 +2149,7 @@ constexpr int kCarrySlots = 16;
 // List entries per particle that the build stages in LDS before writing
 // them row by row; entries past this many go straight to their slot.
 constexpr int kStageSlots = 16;
+static_assert(kStageSlots <= kLevSlots, "every staged entry has a gap class");
 
 struct BuildLds {
   uint32_t key[kCarrySlots][kBlock];
@@ -2193,6 +2299,10 @@ __global__ __launch_bounds__(kBlock) void k_build(RebuildArgs a) {
     const int stage = a.W < kStageSlots ? a.W : kStageSlots;
     uint32_t tmask = 0u;  // staged entries that touch
     int nts = 0;          // their number
+    uint32_t glo = 0u, ghi = 0u;  // the staged entries' gap classes (kReachGap)
+    const double gap1 = p.skin * ((double)kReachGap[1] / kReachUnits),
+                 gap2 = p.skin * ((double)kReachGap[2] / kReachUnits),
+                 gap3 = p.skin * ((double)kReachGap[3] / kReachUnits);
 #pragma unroll
     for (int row = 0; row < 9; row++) {
       const int s0 = cs[3 * row], s1 = cs[3 * row + 1], s2 = cs[3 * row + 2];
@@ -2239,6 +2349,13 @@ __global__ __launch_bounds__(kBlock) void k_build(RebuildArgs a) {
             }
             if (cnt < stage) {
               lds.entry[cnt][t] = entry;
+              // (dev_units rounds up by far more than these products round)
+              if (rsq >= (radsum + gap2) * (radsum + gap2)) {
+                ghi |= 1u << cnt;
+                if (rsq >= (radsum + gap3) * (radsum + gap3)) glo |= 1u << cnt;
+              } else if (rsq >= (radsum + gap1) * (radsum + gap1)) {
+                glo |= 1u << cnt;
+              }
               if (touch) {
                 if (nts < kCarrySlots)
                   lds.carried[nts][t] = (uint16_t)(m + 1);
@@ -2258,7 +2375,7 @@ __global__ __launch_bounds__(kBlock) void k_build(RebuildArgs a) {
     }
     // staged entries, touching ones first, one list row at a time
     const int staged = cnt < stage ? cnt : stage;
-    uint32_t mt = tmask, mn = ~tmask & (staged < 32 ? (1u << staged) - 1u : ~0u);
+    uint32_t mt = tmask, mn = ~tmask & (staged < 32 ? (1u << staged) - 1u : ~0u), lev = 0u;
     for (int s = 0; s < staged; s++) {
       int k;
       if (mt) {
@@ -2269,7 +2386,9 @@ __global__ __launch_bounds__(kBlock) void k_build(RebuildArgs a) {
         mn &= mn - 1u;
       }
       a.newl.nbr[(size_t)s * cap + i] = lds.entry[k][t];
+      lev |= (((glo >> k) & 1u) | (((ghi >> k) & 1u) << kLevSlots)) << s;
     }
+    a.aalt.lev[i] = lev;
     // histories of the carried staged entries, at their touching rank
     const int nq = nts < kCarrySlots ? nts : kCarrySlots;
     for (int q = 0; q < nq; q++) {
@@ -2302,6 +2421,8 @@ __global__ void k_reset_build_counters(Ctrl *ctrl) {
     ctrl->mesh_overflow = 0;
     ctrl->nmesh_cand = 0;
     ctrl->nlost = 0;
+    ctrl->reach = 0;
+    for (int k = 0; k < 6; k++) ctrl->drift[k / 3][k % 3] = 0.0;
   }
 }
 

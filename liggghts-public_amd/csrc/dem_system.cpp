@@ -149,6 +149,7 @@ struct dem_handle {
   // counters
   int64_t ntimestep = 0, nrebuilds = 0;
   int64_t last_build = 0;  // timestep of the last neighbor build
+  int drift_slot = 0;      // Ctrl::drift slot of the last run's final step
   int64_t npairs = 0, ncontacts = 0, nwall_contacts = 0, nmesh_cand = 0;
   int maxcount = 0;
   bool timing = false;
@@ -280,6 +281,9 @@ dem::DevParams make_devparams(const dem_handle *h) {
   d.neigh_every = p.neigh_every > 0 ? p.neigh_every : 1;
   d.neigh_check = p.neigh_no_check ? 0 : 1;
   d.skin = p.skin;
+  // without the displacement check (or a skin) distances are not followed
+  d.reach_on = (d.neigh_check && p.skin > 0.0) ? 1 : 0;
+  d.reach_scale = d.reach_on ? (float)(dem::kReachUnits / p.skin) : 0.f;
   d.cdf = p.cdf;
   d.cdm = p.cdf * p.cdf;
   d.close_band = p.cdf > 1.0 ? 1 : 0;
@@ -887,6 +891,7 @@ int grow_particles(dem_handle *h, int newcap) {
     cols.push_back({(void **)&h->aux[b].tag, sizeof(int), 1, 0, true});
     cols.push_back({(void **)&h->aux[b].orig, sizeof(int), 1, 0, true});
     cols.push_back({(void **)&h->aux[b].meta, sizeof(int), 1, 0, true});
+    cols.push_back({(void **)&h->aux[b].lev, sizeof(uint32_t), 1, 0, true});
     cols.push_back({&h->aux[b].whist, h->fsz, h->hw * nw, 0, true});
     cols.push_back({(void **)&h->aux[b].mslot, sizeof(int), nm * dem::kMeshSlots, 0xff, true});
     cols.push_back({&h->aux[b].mhist, h->fsz, h->hw * nm * dem::kMeshSlots, 0, true});
@@ -1487,6 +1492,7 @@ int dem_set_particles(dem_handle *h, int64_t n, const double *x, const double *v
     if ((rc = dalloc(h, (void **)&h->aux[b].tag, sizeof(int) * cap))) return rc;
     if ((rc = dalloc(h, (void **)&h->aux[b].orig, sizeof(int) * cap))) return rc;
     if ((rc = dalloc(h, (void **)&h->aux[b].meta, sizeof(int) * cap))) return rc;
+    if ((rc = dalloc(h, (void **)&h->aux[b].lev, sizeof(uint32_t) * cap))) return rc;
     if ((rc = dalloc(h, &h->aux[b].whist, h->fsz * h->hw * nw * cap))) return rc;
     if ((rc = dalloc(h, (void **)&h->lst[b].nbr, sizeof(uint32_t) * h->W * cap))) return rc;
     if ((rc = dalloc(h, &h->lst[b].hist, h->fsz * dem::hist_rec(h->hw) * h->W * cap))) return rc;
@@ -1806,6 +1812,7 @@ int run_steps_piece(dem_handle *h, int64_t nsteps) {
   if (h->n > 0) {
     dem::StepArgs a = step_args(h, h->cur_st, h->tri_cur);
     a.ago_next = ts0 + 1 - h->last_build;
+    a.drift_from = h->drift_slot;
     HIPCHK(h, dem::launch_initial(a, h->stream));
   }
   // the inserted particles: after the initial integrate of the others, before
@@ -1916,6 +1923,7 @@ int run_steps_piece(dem_handle *h, int64_t nsteps) {
     }
   }
   h->tri_cur = tc;
+  h->drift_slot = (int)(nsteps & 1);
   if (timed) h->mesh_time = t_end;
   h->pending_mesh_rebuild = h->ctrl_host->stop_at == nsteps + 1;
   h->ncontacts = (int64_t)(h->ctrl_host->ncontact_full / 2);
@@ -2265,6 +2273,8 @@ int dem_read_restart(dem_handle *h, const char *path) {
   }
   fclose(f);
   if (!ok) return fail(h, DEM_ERR_ARG, "read_restart: truncated file");
+  // the rows' gap classes are not in the file: they are walked whole until the next build
+  HIPCHK(h, hipMemset(h->aux[h->cur_aux].lev, 0, sizeof(uint32_t) * (size_t)h->cap));
   h->have_list = hd.have_list != 0;
   h->pending_mesh_rebuild = hd.pending_mesh_rebuild != 0;
   h->ntimestep = hd.ntimestep;
