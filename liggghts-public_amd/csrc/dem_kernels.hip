@@ -25,13 +25,27 @@ constexpr double kPi = 3.14159265358979323846;  // M_PI
 // ---------------------------------------------------------------------------
 
 // Workgroups are dispatched round-robin over the 8 XCDs (block b -> XCD b%8).
-// Remap so that each XCD walks one contiguous range of Morton-ordered
-// particles: neighbors of a particle then sit in the same XCD's L2.
+// Remap so that each XCD walks stretches of kXcdChunk consecutive tiles of
+// Morton-ordered particles: the neighbors of a particle then mostly sit in the
+// same XCD's L2 (a stretch's records are under 1 MB of its 4), and the
+// stretches of the XCDs alternate, so that a region with more contacts than
+// the rest (the bottom of a filling) is spread over all of them. One contiguous
+// eighth per XCD left most of the chip waiting for the eighths at the bottom:
+// 700 steps of 1M spheres settling with 270k contacts, mixed 76 -> 59 ms, FP64
+// 108 -> 81 ms; stretches of 4 and 64 tiles measured within 5 % of 16.
+constexpr int kXcdChunk = 16;
 __device__ __forceinline__ int xcd_block(int nblocks) {
   const int b = blockIdx.x;
-  const int xcd = b & 7, slot = b >> 3;
-  const int q = nblocks >> 3, r = nblocks & 7;
-  return xcd * q + (xcd < r ? xcd : r) + slot;
+  const int whole = nblocks / (8 * kXcdChunk) * (8 * kXcdChunk);
+  if (b < whole) {
+    const int xcd = b & 7, slot = b >> 3;
+    return ((slot / kXcdChunk) * 8 + xcd) * kXcdChunk + slot % kXcdChunk;
+  }
+  // the rest: one stretch per XCD
+  const int r = b - whole, n = nblocks - whole;
+  const int xcd = r & 7, slot = r >> 3;
+  const int q = n >> 3, m = n & 7;
+  return whole + xcd * q + (xcd < m ? xcd : m) + slot;
 }
 
 __device__ __forceinline__ int cell_coord(const DevParams &p, int d, double x) {
