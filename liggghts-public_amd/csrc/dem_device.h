@@ -53,6 +53,14 @@ constexpr int kStepVariantBlock[kNumStepVariants] = {256, 256, 256, 128, 64, 256
 constexpr int kStepVariantGroup[kNumStepVariants] = {4, 2, 8, 4, 4, 4, 8, 4, 8, 4, 4};
 constexpr int kStepVariantWave[kNumStepVariants] = {0, 0, 0, 0, 0, 1, 1, 2, 2, 3, 3};
 
+// Lane groups: a small system in shape 0 steps each particle with 4 or 8
+// lanes of a wavefront (StepArgs::lanes), in blocks of one wavefront so that
+// the few there are spread over the chip.
+constexpr int kGroupBlock = 64;
+constexpr int step_block(int variant, int lanes) {
+  return lanes > 1 ? kGroupBlock : kStepVariantBlock[variant];
+}
+
 // One triangle of a fix mesh/surface, FP64 (TriMesh element properties).
 struct TriGeom {
   double n[9];   // nodes
@@ -254,6 +262,7 @@ struct StepArgs {
   // moving meshes, blocks [pblocks, gridDim) rotate the meshes into the next
   // step's geometry buffer (mv.dst) while the others compute this step
   int variant, pblocks, move_mesh;
+  int lanes;           // lanes per particle (1, or 4 or 8 in shape 0)
   int drift_from;      // k_initial: the drift slot of the last run's final step
   int step_from_ctrl;  // step = ctrl->step_base + step, ago_next = ctrl->ago_base + step
   MeshMoveArgs mv;

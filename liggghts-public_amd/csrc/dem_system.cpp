@@ -433,6 +433,33 @@ dem::RebuildArgs rebuild_args(dem_handle *h) {
 
 dem::MeshMoveArgs mesh_move_args(const dem_handle *h, long long step, int guard, int decide);
 
+// the sibling models run in shapes 0 and 5 only
+int step_variant(const dem_handle *h) {
+  return ((uses_generic_models(h) || h->hw != 3) && h->variant != 5) ? 0 : h->variant;
+}
+
+// Lanes per particle in the default shape. One lane resolves a particle's
+// contacts one after another (about 20 us for a bed's six), and that chain is
+// the step when there are too few wavefronts to hide it; a group of lanes takes
+// them together, but spends most of its lanes on what is done once per
+// particle, so it loses as soon as the chip is full. A step of a packed bed
+// in us with 1 / 4 / 8 lanes, hertz mixed and hooke + sjkr FP64:
+//    4,000 spheres  25.8 / 14.2 / 12.4   34.3 / 17.9 / 14.3
+//   12,000          24.7 / 15.1 / 13.9   32.7 / 18.7 / 16.9
+//   24,000          24.6 / 17.1 / 16.7   31.9 / 22.7 / 26.0
+//   48,000          25.7 / 21.2 / 26.3   34.2 / 33.3 / 39.2
+//   80,000          30.9 / 31.6 / 39.0   42.8 / 46.2 / 58.4
+// A cloud without contacts has no chain to shorten (4,000: 10.7 / 9.6 / 9.9,
+// 12,000: 9.0 / 8.7 / 9.3, 24,000: 8.6 / 9.2 / 9.9), so the list's length
+// decides as well.
+int step_lanes(const dem_handle *h) {
+  constexpr int64_t kFew = 16 * 1024, kSome = 48 * 1024;
+  if (step_variant(h) != 0 || h->persist != 0 || h->n > kSome) return 1;
+  const bool packed = h->npairs >= 3 * h->n;  // a row holds six entries or more
+  if (h->n <= kFew) return packed ? 8 : 4;
+  return packed ? 4 : 1;
+}
+
 // in_buf: particle state buffer read by the step; tri_buf: geometry buffer of
 // the step (the next step's geometry goes to the other one)
 dem::StepArgs step_args(dem_handle *h, int in_buf, int tri_buf) {
@@ -456,10 +483,10 @@ dem::StepArgs step_args(dem_handle *h, int in_buf, int tri_buf) {
   a.fout = h->fout;
   a.ctrl = h->ctrl;
   a.inst_stats = h->d_inst_stats;
-  // the sibling models run in shapes 0 and 5 only
-  a.variant = (a.prm.generic && h->variant != 5) ? 0 : h->variant;
+  a.variant = step_variant(h);
+  a.lanes = step_lanes(h);
   {
-    const int B = dem::kStepVariantBlock[a.variant];
+    const int B = dem::step_block(a.variant, a.lanes) / a.lanes;
     const int ntiles = (int)((std::max<int64_t>(h->n, 1) + B - 1) / B);
     a.pblocks = h->persist > 0 ? std::min(ntiles, h->persist * h->ncu) : ntiles;
   }
@@ -1712,7 +1739,7 @@ constexpr int kGraphBatch = 32; // steps per captured graph
 // take their step index from the control block (launch_set_base).
 int step_graph(dem_handle *h, int st, int tc, bool moving, hipGraphExec_t *out) {
   const int key = st | (tc << 1) | (h->cur_aux << 2) | (h->variant << 3) | (h->persist << 6) |
-                  ((moving ? 1 : 0) << 13);
+                  ((moving ? 1 : 0) << 13) | (step_lanes(h) << 14);
   for (auto &g : h->graphs)
     if (g.key == key) {
       *out = g.exec;
