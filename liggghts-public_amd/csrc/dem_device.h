@@ -37,6 +37,8 @@ constexpr int kReachGap[4] = {0, 32, 88, 176};
 constexpr int kMaxMeshes = 4;
 constexpr int kMeshSlots = 8;       // contact-history slots per particle and mesh
 constexpr int kMaxMeshCand = 32;    // candidate triangles per particle (all meshes)
+constexpr int kMeshBlock = 64;      // k_step_mesh: threads per block ...
+constexpr int kMeshBlocks = 1024;   // ... and blocks at most: a wavefront per SIMD
 // omega.w of a particle holds type + (instance << kTypeBits): independent
 // simulations batched in one system each own a cell grid and a material block
 constexpr int kTypeBits = 8;
@@ -163,7 +165,8 @@ struct Ctrl {
   unsigned long long nlost;  // atoms beyond an f face at the last build
   // since the last build: the largest distance of a particle (kMetaDevShift),
   // and the drift it is taken from, of steps of even and odd index
-  int reach, pad3;
+  int reach;
+  int nmesh_near;  // particles with candidate triangles at the last build (MeshStep::near)
   double drift[2][3];
 };
 
@@ -192,6 +195,7 @@ struct MeshStep {
   const int *copl_off, *copl_idx;  // coplanar node-neighbor lists per triangle
   const int *cand;                 // [kMaxMeshCand][cap] candidate triangles, ascending
   const int *ncand;                // [cap]
+  const int *near;                 // [cap] the particles with candidates, packed
 };
 
 struct ListBuf {
@@ -294,7 +298,7 @@ struct RebuildArgs {
   int *tpair_cell, *tpair_tri; // triangle-cell pairs
   int tpair_cap;
   int *tcell_count, *tcell_start, *tcell_list;
-  int *cand, *ncand;
+  int *cand, *ncand, *near;
   int zero_vnode;              // setup: node velocities start at zero
 };
 

@@ -13,6 +13,7 @@
 // The file is compiled with -ffp-contract=off: in FP64 mode every product and
 // sum rounds as in the CPU reference, so one pair's contribution is bitwise
 // equal to the reference's; only the order of the per-particle sums differs.
+#include <algorithm>
 #include <type_traits>
 
 #include "dem_device.h"
@@ -514,6 +515,10 @@ __device__ __forceinline__ void mesh_contacts(const StepArgs &a, int i, const do
     const bool roll = GEN && mdl.epsd2;
     const int mt = irow + p.mesh_wtype[m];
     unsigned keep = 0u;
+    // the slots, read at once: looked up one by one they are a chain of loads
+    int held[kMeshSlots];
+#pragma unroll
+    for (int k = 0; k < kMeshSlots; k++) held[k] = slot[(size_t)k * cap];
     for (; c < nc; c++) {
       const int t = M.cand[(size_t)c * cap + i];
       if (t >= tend) break;
@@ -526,32 +531,29 @@ __device__ __forceinline__ void mesh_contacts(const StepArgs &a, int i, const do
       if (!(deltan <= 0 || deltan < (p.cdf - 1.0) * pi.w)) continue;
       // handleContact
       int s = -1;
-      for (int k = 0; k < kMeshSlots; k++)
-        if (slot[(size_t)k * cap] == t) {
-          s = k;
-          break;
-        }
+#pragma unroll
+      for (int k = kMeshSlots - 1; k >= 0; k--) s = held[k] == t ? k : s;
       bool fresh = false;
       if (s >= 0) {
         keep |= 1u << s;
       } else {
         bool skip = false;
         if (bs == 7)
+#pragma unroll
           for (int k = 0; k < kMeshSlots; k++) {
-            const int st = slot[(size_t)k * cap];
+            const int st = held[k];
             if (st >= 0 && st != t && ((keep >> k) & 1u) && tri_coplanar(M, st, t)) skip = true;
           }
         if (skip) continue;
-        for (int k = 0; k < kMeshSlots; k++)
-          if (slot[(size_t)k * cap] == -1) {
-            s = k;
-            break;
-          }
+#pragma unroll
+        for (int k = kMeshSlots - 1; k >= 0; k--) s = held[k] == -1 ? k : s;
         if (s < 0) {
           atomicMax(&a.ctrl->slot_overflow, 1);
           continue;
         }
         slot[(size_t)s * cap] = t;
+#pragma unroll
+        for (int k = 0; k < kMeshSlots; k++) held[k] = k == s ? t : held[k];
         keep |= 1u << s;
         fresh = true;
       }
@@ -559,8 +561,9 @@ __device__ __forceinline__ void mesh_contacts(const StepArgs &a, int i, const do
       if (fresh) {
         sh[0] = sh[1] = sh[2] = T(0);
         if (bs == 7)  // checkCoplanarContactHistory: the last coplanar slot wins
+#pragma unroll
           for (int k = 0; k < kMeshSlots; k++) {
-            const int st = slot[(size_t)k * cap];
+            const int st = held[k];
             if (st >= 0 && st != t && tri_coplanar(M, st, t))
               for (int d = 0; d < 3; d++) {
                 sh[d] = hist[(size_t)(k * mhw + d) * cap];
@@ -660,8 +663,9 @@ __device__ __forceinline__ void mesh_contacts(const StepArgs &a, int i, const do
         }
     }
     // cleanUpContacts: slots not touched this pass are freed
+#pragma unroll
     for (int k = 0; k < kMeshSlots; k++)
-      if (!((keep >> k) & 1u) && slot[(size_t)k * cap] != -1) slot[(size_t)k * cap] = -1;
+      if (!((keep >> k) & 1u) && held[k] != -1) slot[(size_t)k * cap] = -1;
   }
 }
 
@@ -1521,12 +1525,15 @@ __device__ __forceinline__ void step_particle(const StepArgs &a, const int i, co
       }
     }
   }
+  const size_t cap = (size_t)a.cap;
+  // a particle with candidate triangles is left to k_step_mesh after the walls
+  const bool near_mesh = MESH && a.mesh.ncand[i] != 0;
   // post_force fixes in script order: gravity (fix_gravity.cpp:331-338) and
   // plane walls (fix_wall_gran.cpp:1024-1153)
   for (int pass = 0; pass < 2; pass++) {
     const bool grav_pass = (pass == 0) == (p.grav_first != 0);
     if (grav_pass) {
-      if (p.has_grav) {
+      if (p.has_grav && !(MESH && near_mesh && !p.grav_first)) {
         fx += (T)(vi.w * p.gacc[0]);
         fy += (T)(vi.w * p.gacc[1]);
         fz += (T)(vi.w * p.gacc[2]);
@@ -1550,10 +1557,18 @@ __device__ __forceinline__ void step_particle(const StepArgs &a, const int i, co
         meta &= ~bit;  // history zeroed when the contact ends (fix_wall_gran.cpp:1145-1151)
       }
     }
-    if (MESH)
-      mesh_contacts<T, GEN>(a, i, pi, vi, wi, irow, fx, fy, fz, tx, ty, tz, my_wall);
   }
 
+  if (MESH && near_mesh) {
+    a.fout[i] = (double)fx;
+    a.fout[cap + i] = (double)fy;
+    a.fout[2 * cap + i] = (double)fz;
+    a.fout[3 * cap + i] = (double)tx;
+    a.fout[4 * cap + i] = (double)ty;
+    a.fout[5 * cap + i] = (double)tz;
+    if (meta != meta0) a.aux.meta[i] = meta;
+    return;
+  }
   finish_particle<T>(a, i, pi, vi, wi, fx, fy, fz, tx, ty, tz, meta, displaced, dev, drift, ago_next);
   if (meta != meta0) a.aux.meta[i] = meta;
 }
@@ -1744,75 +1759,41 @@ __device__ __forceinline__ void step_group(const StepArgs &a, const int i,
   }
 }
 
-// ---------------------------------------------------------------------------
-// fused step kernel: pair forces over the full list, plane walls, meshes,
-// gravity, nve/sphere final integrate of this step and initial integrate of
-// the next, and the skin/2 displacement check of Neighbor::decide for the
-// next step. One thread per particle in tiles of BLOCK particles; the
-// first pblocks blocks walk the tiles (one tile each, or several when the
-// grid is made persistent). With moving meshes, trailing blocks rotate the
-// meshes into the next step's geometry buffer. Every tile shape computes
-// the same arithmetic in the same order, so results do not depend on it.
-// ---------------------------------------------------------------------------
-template <typename T, bool MESH, int BLOCK, int GROUP, bool GEN = false, int WAVE = 0, int LANES = 1>
-__global__ __launch_bounds__(BLOCK) void k_step(StepArgs a) {
-  // in a captured graph the step index is the control block's base plus this
-  // launch's offset (a.step)
-  long long step = a.step, ago_next = a.ago_next;
+// In a captured graph the step index is the control block's base plus the
+// launch's offset (a.step). False: a rebuild is due first.
+__device__ __forceinline__ bool step_index(const StepArgs &a, long long &step, long long &ago_next) {
+  step = a.step;
+  ago_next = a.ago_next;
   if (a.step_from_ctrl) {
     step = a.ctrl->step_base + a.step;
     ago_next = a.ctrl->ago_base + a.step;
   }
-  if (step >= a.ctrl->stop_at) return;
-  if (MESH && (int)blockIdx.x >= a.pblocks) {
-    mesh_move_block(a.mv, ((int)blockIdx.x - a.pblocks) * BLOCK + threadIdx.x, step + 1);
-    return;
-  }
-  const DevParams &p = a.prm;
-  constexpr bool kGrouped = LANES > 1;
-  typedef typename std::conditional<kGrouped, GroupLds<T>, typename PairLdsT<T, GROUP, WAVE>::type>::type Lds;
-  constexpr bool kWaveLds = WAVE == 1 || WAVE == 2 || kGrouped;
-  __shared__ Lds lds_all[kWaveLds ? BLOCK / 64 : 1];
-  Lds *lds = &lds_all[kWaveLds ? (threadIdx.x >> 6) : 0];
-  unsigned long long my_contacts = 0, my_wall = 0;
-  bool displaced = false;
-  // the drift the particles' distances are taken from: one particle's path
-  // since the build, so that a cloud moving as one keeps its rows' reach. Any
-  // common vector serves; it is advanced by that particle's velocity as it
-  // stands in this launch's input, which every wavefront reads alike.
-  int dev = 0;
-  const int reach = a.ctrl->reach;
-  double drift[3] = {0.0, 0.0, 0.0};
-  if (p.reach_on && a.do_initial) {
+  return step < a.ctrl->stop_at;
+}
+
+// The drift the particles' distances are taken from: one particle's path since
+// the build, so that a cloud moving as one keeps its rows' reach. Any common
+// vector serves; it is advanced by that particle's velocity as it stands in
+// this step's input, which every wavefront reads alike.
+__device__ __forceinline__ void step_drift(const StepArgs &a, const long long step, double drift[3]) {
+  drift[0] = drift[1] = drift[2] = 0.0;
+  if (a.prm.reach_on && a.do_initial) {
     const double *d0 = a.ctrl->drift[step & 1];
     const double4 v = a.in.vel[a.n >> 1];
-    drift[0] = d0[0] + p.dt * v.x;
-    drift[1] = d0[1] + p.dt * v.y;
-    drift[2] = d0[2] + p.dt * v.z;
-    if (blockIdx.x == 0 && threadIdx.x < 3) a.ctrl->drift[(step + 1) & 1][threadIdx.x] = drift[threadIdx.x];
+    drift[0] = d0[0] + a.prm.dt * v.x;
+    drift[1] = d0[1] + a.prm.dt * v.y;
+    drift[2] = d0[2] + a.prm.dt * v.z;
   }
-  constexpr int TILE = BLOCK / LANES;
-  const int ntiles = (a.n + TILE - 1) / TILE;
-  for (int tile = xcd_block(a.pblocks); tile < ntiles; tile += a.pblocks) {
-    const int i = tile * TILE + (int)threadIdx.x / LANES;
-    const bool active = i < a.n;
-    if ((kWaveLds && !kGrouped) || active) {
-      unsigned long long c = 0, w = 0;
-      int inst = 0;
-      if constexpr (kGrouped)
-        step_group<T, MESH, GEN, LANES>(a, i, c, w, inst, displaced, dev, reach, drift, ago_next, *lds);
-      else
-        step_particle<T, MESH, GROUP, GEN, WAVE>(a, i, active, c, w, inst, displaced, dev, reach, drift, ago_next, lds);
-      my_contacts += c;
-      my_wall += w;
-      if (active && a.count && a.inst_stats) {
-        if (c) atomicAdd(&a.inst_stats[inst], c);
-        if (w) atomicAdd(&a.inst_stats[p.ninst + inst], w);
-      }
-    }
-  }
+}
 
-  if (p.reach_on && a.do_initial) raise_reach(a.ctrl, dev, reach);
+// What a block's particles ask for: the reach raised, a rebuild before the
+// next step, the contact counts.
+template <int BLOCK>
+__device__ __forceinline__ void step_end(const StepArgs &a, const long long step,
+                                         const unsigned long long my_contacts,
+                                         const unsigned long long my_wall, const bool displaced,
+                                         const int dev, const int reach) {
+  if (a.prm.reach_on && a.do_initial) raise_reach(a.ctrl, dev, reach);
   // rebuild request for the next step
   if (__ballot(displaced) != 0ull) {
     if ((threadIdx.x & 63) == 0)
@@ -1840,6 +1821,122 @@ __global__ __launch_bounds__(BLOCK) void k_step(StepArgs a) {
       if (tw) atomicAdd(&a.ctrl->nwall, tw);
     }
   }
+}
+
+// ---------------------------------------------------------------------------
+// fused step kernel: pair forces over the full list, plane walls, meshes,
+// gravity, nve/sphere final integrate of this step and initial integrate of
+// the next, and the skin/2 displacement check of Neighbor::decide for the
+// next step. One thread per particle in tiles of BLOCK particles; the
+// first pblocks blocks walk the tiles (one tile each, or several when the
+// grid is made persistent). With moving meshes, trailing blocks rotate the
+// meshes into the next step's geometry buffer. Every tile shape computes
+// the same arithmetic in the same order, so results do not depend on it.
+// ---------------------------------------------------------------------------
+// With a mesh the mixed kernel comes to 129 registers, one over what leaves room
+// for four wavefronts per SIMD; asked for four, it takes 128 and spills none.
+template <typename T, bool MESH, int GROUP, bool GEN, int WAVE, int LANES>
+constexpr bool kFourWaves = MESH && sizeof(T) == 4 && GROUP <= 4 && !GEN && WAVE == 0 && LANES == 1;
+template <typename T, bool MESH, int BLOCK, int GROUP, bool GEN = false, int WAVE = 0, int LANES = 1>
+__global__ __launch_bounds__(BLOCK)
+    __attribute__((amdgpu_waves_per_eu(kFourWaves<T, MESH, GROUP, GEN, WAVE, LANES> ? 4 : 1))) void k_step(StepArgs a) {
+  long long step, ago_next;
+  if (!step_index(a, step, ago_next)) return;
+  if (MESH && (int)blockIdx.x >= a.pblocks) {
+    mesh_move_block(a.mv, ((int)blockIdx.x - a.pblocks) * BLOCK + threadIdx.x, step + 1);
+    return;
+  }
+  const DevParams &p = a.prm;
+  constexpr bool kGrouped = LANES > 1;
+  typedef typename std::conditional<kGrouped, GroupLds<T>, typename PairLdsT<T, GROUP, WAVE>::type>::type Lds;
+  constexpr bool kWaveLds = WAVE == 1 || WAVE == 2 || kGrouped;
+  __shared__ Lds lds_all[kWaveLds ? BLOCK / 64 : 1];
+  Lds *lds = &lds_all[kWaveLds ? (threadIdx.x >> 6) : 0];
+  unsigned long long my_contacts = 0, my_wall = 0;
+  bool displaced = false;
+  int dev = 0;
+  const int reach = a.ctrl->reach;
+  double drift[3];
+  step_drift(a, step, drift);
+  if (p.reach_on && a.do_initial && blockIdx.x == 0 && threadIdx.x < 3)
+    a.ctrl->drift[(step + 1) & 1][threadIdx.x] = drift[threadIdx.x];
+  constexpr int TILE = BLOCK / LANES;
+  const int ntiles = (a.n + TILE - 1) / TILE;
+  for (int tile = xcd_block(a.pblocks); tile < ntiles; tile += a.pblocks) {
+    const int i = tile * TILE + (int)threadIdx.x / LANES;
+    const bool active = i < a.n;
+    if ((kWaveLds && !kGrouped) || active) {
+      unsigned long long c = 0, w = 0;
+      int inst = 0;
+      if constexpr (kGrouped)
+        step_group<T, MESH, GEN, LANES>(a, i, c, w, inst, displaced, dev, reach, drift, ago_next, *lds);
+      else
+        step_particle<T, MESH, GROUP, GEN, WAVE>(a, i, active, c, w, inst, displaced, dev, reach, drift, ago_next, lds);
+      my_contacts += c;
+      my_wall += w;
+      if (active && a.count && a.inst_stats) {
+        if (c) atomicAdd(&a.inst_stats[inst], c);
+        if (w) atomicAdd(&a.inst_stats[p.ninst + inst], w);
+      }
+    }
+  }
+
+  step_end<BLOCK>(a, step, my_contacts, my_wall, displaced, dev, reach);
+}
+
+// The rest of the step of the particles with candidate triangles: k_step left
+// the sum of their pairs, walls and (where it comes first) gravity in fout.
+// They are a few percent of a system and sit in most of its wavefronts, so in
+// k_step every wavefront paid for a triangle search and a contact law that one
+// lane in twenty used, and all of it for their registers (202, two wavefronts
+// per SIMD; 127 and four without). Here they are packed, from the list of the
+// last build, in no particular order: no particle depends on another. Bound by
+// latency, 15 to 20 us whatever their number. A step in us, the mesh in k_step
+// / here (k_step + k_step_mesh): 727k spheres in 48 heaps on a floor, mixed,
+// 90 / 55 + 15; 250k in a drum, 64 / 44 + 20. In leading blocks of k_step's own
+// launch, whose registers then spill, the two came to 93 and 64.
+template <typename T, bool GEN>
+__global__ __launch_bounds__(kMeshBlock) void k_step_mesh(StepArgs a) {
+  typedef typename OmgT<T>::type omg_t;
+  const DevParams &p = a.prm;
+  long long step, ago_next;
+  if (!step_index(a, step, ago_next)) return;
+  unsigned long long my_wall = 0;
+  bool displaced = false;
+  int dev = 0;
+  const int reach = a.ctrl->reach, listed = a.ctrl->nmesh_near;
+  double drift[3];
+  step_drift(a, step, drift);
+  const size_t cap = (size_t)a.cap;
+  // spread over all the blocks, a few lanes of each: there are too few to fill
+  // the chip, and a wavefront walks every case its triangles fall into
+  const int per = (listed + (int)gridDim.x - 1) / (int)gridDim.x;
+  const int last = std::min(listed, ((int)blockIdx.x + 1) * per);
+  for (int k = (int)blockIdx.x * per + (int)threadIdx.x; k < last; k += kMeshBlock) {
+    const int i = a.mesh.near[k];
+    const double4 pi = a.in.pos[i];
+    const double4 vi = a.in.vel[i];
+    const omg_t wi = ((const omg_t *)a.in.omg)[i];
+    const int wbits = (int)wi.w;
+    const int inst = wbits >> kTypeBits;
+    const int irow = inst * p.mat_stride + (wbits & kTypeMask) * p.ntp1;
+    const int meta0 = a.aux.meta[i];
+    int meta = meta0;
+    T fx = (T)a.fout[i], fy = (T)a.fout[cap + i], fz = (T)a.fout[2 * cap + i];
+    T tx = (T)a.fout[3 * cap + i], ty = (T)a.fout[4 * cap + i], tz = (T)a.fout[5 * cap + i];
+    unsigned long long w = 0;
+    mesh_contacts<T, GEN>(a, i, pi, vi, wi, irow, fx, fy, fz, tx, ty, tz, w);
+    if (p.has_grav && !p.grav_first) {
+      fx += (T)(vi.w * p.gacc[0]);
+      fy += (T)(vi.w * p.gacc[1]);
+      fz += (T)(vi.w * p.gacc[2]);
+    }
+    finish_particle<T>(a, i, pi, vi, wi, fx, fy, fz, tx, ty, tz, meta, displaced, dev, drift, ago_next);
+    if (meta != meta0) a.aux.meta[i] = meta;
+    my_wall += w;
+    if (a.count && a.inst_stats && w) atomicAdd(&a.inst_stats[p.ninst + inst], w);
+  }
+  step_end<kMeshBlock>(a, step, 0, my_wall, displaced, dev, reach);
 }
 
 // compute pair/gran/local (compute_pair_gran_local.cpp:312-470) through
@@ -2659,6 +2756,7 @@ __global__ void k_reset_build_counters(Ctrl *ctrl) {
     ctrl->npairs_full = 0;
     ctrl->mesh_overflow = 0;
     ctrl->nmesh_cand = 0;
+    ctrl->nmesh_near = 0;
     ctrl->nlost = 0;
     ctrl->reach = 0;
     for (int k = 0; k < 6; k++) ctrl->drift[k / 3][k % 3] = 0.0;
@@ -2891,6 +2989,19 @@ __global__ __launch_bounds__(kBlock) void k_mesh_cand(RebuildArgs a) {
   if ((threadIdx.x & 63) == 0 && nc) atomicAdd(&a.ctrl->nmesh_cand, nc);
 }
 
+// The particles with candidate triangles, packed.
+__global__ __launch_bounds__(kBlock) void k_mesh_near(RebuildArgs a) {
+  const int i = blockIdx.x * kBlock + threadIdx.x;
+  const int lane = threadIdx.x & 63;
+  const bool near = i < a.n && a.ncand[i] != 0;
+  const unsigned long long m = __ballot(near);
+  if (m == 0ull) return;
+  int at = 0;
+  if (lane == 0) at = atomicAdd(&a.ctrl->nmesh_near, __popcll(m));
+  at = __shfl(at, 0, 64);
+  if (near) a.near[at + __popcll(m & ((1ull << lane) - 1ull))] = i;
+}
+
 // the first step of a run: meshes rotated in place
 __global__ __launch_bounds__(kBlock) void k_mesh_move(MeshMoveArgs a) {
   if (a.guard && a.step >= a.ctrl->stop_at) return;
@@ -3064,6 +3175,22 @@ hipError_t launch_step(const StepArgs &a, hipStream_t s) {
     else
       launch_step_variant<double, false>(a, nb, s);
   }
+  // one lane per particle leaves the particles near a mesh to a launch of
+  // their own, whose grid does not depend on how many the last build found
+  if (mesh && a.lanes == 1) {
+    const dim3 g(std::min(a.n, kMeshBlocks)), b(kMeshBlock);
+    if (a.mixed) {
+      if (a.prm.generic)
+        hipLaunchKernelGGL((k_step_mesh<float, true>), g, b, 0, s, a);
+      else
+        hipLaunchKernelGGL((k_step_mesh<float, false>), g, b, 0, s, a);
+    } else {
+      if (a.prm.generic)
+        hipLaunchKernelGGL((k_step_mesh<double, true>), g, b, 0, s, a);
+      else
+        hipLaunchKernelGGL((k_step_mesh<double, false>), g, b, 0, s, a);
+    }
+  }
   return hipGetLastError();
 }
 
@@ -3172,6 +3299,7 @@ hipError_t launch_mesh_bin_fill(const RebuildArgs &a, hipStream_t s) {
       hipLaunchKernelGGL(k_mesh_cand<float>, dim3(nblk(a.n, kBlock)), dim3(kBlock), 0, s, a);
     else
       hipLaunchKernelGGL(k_mesh_cand<double>, dim3(nblk(a.n, kBlock)), dim3(kBlock), 0, s, a);
+    hipLaunchKernelGGL(k_mesh_near, dim3(nblk(a.n, kBlock)), dim3(kBlock), 0, s, a);
   }
   return hipGetLastError();
 }

@@ -109,7 +109,7 @@ struct dem_handle {
   int *d_tpair_cell = nullptr, *d_tpair_tri = nullptr, *d_tcell_list = nullptr;
   int tpair_cap = 0;
   int *d_tcell_count = nullptr, *d_tcell_start = nullptr;
-  int *d_cand = nullptr, *d_ncand = nullptr;
+  int *d_cand = nullptr, *d_ncand = nullptr, *d_near = nullptr;
   int *d_total = nullptr;
   int *h_total = nullptr;  // pinned
   bool zero_vnode = false;
@@ -246,7 +246,7 @@ void free_particles(dem_handle *h) {
   h->d_copl_off = h->d_copl_idx = nullptr;
   h->d_tcount = h->d_toff = h->d_tpair_cell = h->d_tpair_tri = h->d_tcell_list = nullptr;
   h->tpair_cap = 0;
-  h->d_tcell_count = h->d_tcell_start = h->d_cand = h->d_ncand = h->d_total = nullptr;
+  h->d_tcell_count = h->d_tcell_start = h->d_cand = h->d_ncand = h->d_near = h->d_total = nullptr;
   h->cell_rank = h->cell_count = h->cell_start = nullptr;
   h->key = h->perm = h->scan_tmp = nullptr;
   h->ncell = 0;
@@ -427,6 +427,7 @@ dem::RebuildArgs rebuild_args(dem_handle *h) {
   a.tcell_list = h->d_tcell_list;
   a.cand = h->d_cand;
   a.ncand = h->d_ncand;
+  a.near = h->d_near;
   a.zero_vnode = h->zero_vnode ? 1 : 0;
   return a;
 }
@@ -479,6 +480,7 @@ dem::StepArgs step_args(dem_handle *h, int in_buf, int tri_buf) {
   a.mesh.copl_idx = h->d_copl_idx;
   a.mesh.cand = h->d_cand;
   a.mesh.ncand = h->d_ncand;
+  a.mesh.near = h->d_near;
   a.xhold = h->xhold;
   a.fout = h->fout;
   a.ctrl = h->ctrl;
@@ -931,6 +933,7 @@ int grow_particles(dem_handle *h, int newcap) {
   cols.push_back({(void **)&h->perm, sizeof(int), 1, 0, false});
   cols.push_back({(void **)&h->d_cand, sizeof(int), dem::kMaxMeshCand, 0, true});
   cols.push_back({(void **)&h->d_ncand, sizeof(int), 1, 0, true});
+  cols.push_back({(void **)&h->d_near, sizeof(int), 1, 0, true});
   int rc;
   for (Col &c : cols) {
     void *np = nullptr;
@@ -1571,6 +1574,7 @@ int dem_set_particles(dem_handle *h, int64_t n, const double *x, const double *v
   }
   if ((rc = dalloc(h, (void **)&h->d_cand, sizeof(int) * dem::kMaxMeshCand * cap))) return rc;
   if ((rc = dalloc(h, (void **)&h->d_ncand, sizeof(int) * cap))) return rc;
+  if ((rc = dalloc(h, (void **)&h->d_near, sizeof(int) * cap))) return rc;
   HIPCHK(h, hipMemset(h->d_ncand, 0, sizeof(int) * cap));
   h->d_inst_stats = nullptr;
   if (h->ninst > 1) {
@@ -1605,6 +1609,8 @@ int dem_set_particles(dem_handle *h, int64_t n, const double *x, const double *v
   HIPCHK(h, hipMemcpy(h->aux[0].orig, orig.data(), sizeof(int) * n, hipMemcpyHostToDevice));
   HIPCHK(h, hipMemcpy(h->aux[0].meta, zero.data(), sizeof(int) * n, hipMemcpyHostToDevice));
   HIPCHK(h, hipMemset(h->fout, 0, sizeof(double) * 6 * cap));
+  // no particle is near a mesh until the first build (d_ncand is zero)
+  HIPCHK(h, hipMemset(&h->ctrl->nmesh_near, 0, sizeof(int)));
   h->cur_st = h->cur_aux = h->cur_l = 0;
   h->have_list = false;
   h->setup_done = false;
