@@ -20,7 +20,8 @@
 //   - lane c owns column c of the Jacobian and forms the four cofactors of
 //     row c of its inverse.
 // Values move inside a row of 16 lanes by DPP (quad_perm, row_ror:8); no LDS.
-// 100k fresh pairs: 232 -> 19 ms; k_pairs of 50k superquadrics 43 -> 4.0 ms a step.
+// An iteration takes 2.7 us. 100k fresh pairs: 126 -> 21 ms to 228 -> 33 ms by
+// the slowest pair drawn; k_pairs of 50k superquadrics 43 -> 7.4 ms a step.
 #pragma once
 
 #include "sq_device.h"

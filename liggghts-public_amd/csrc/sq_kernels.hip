@@ -1,5 +1,5 @@
 // Superquadric contact points on the GPU: the FP64 Newton solve for many
-// independent pose pairs (one thread each), and the contact-point network
+// independent pose pairs (eight lanes each), and the contact-point network
 // that warm-starts it -- an 18 -> 64 -> 64 -> 3 tanh MLP whose forward and
 // backward passes run on BF16 matrix cores (v_mfma_f32_16x16x16_bf16) with
 // FP32 accumulation, trained here with Adam on FP32 master weights.

@@ -6,7 +6,8 @@
 // Data: per-particle arrays in the caller's order (the expensive part is the
 // per-pair Newton solve, not the particle streams, so no reordering); a half
 // pair list (i < j) in CSR form by i with j ascending, and the same pairs
-// listed by j. The pair kernel runs one thread per pair and writes a force
+// listed by j. The pairs whose contact point has to be solved are queued for
+// groups of eight lanes; then one thread per pair writes a force
 // record (force on i, torque on i, torque on j); the gather kernel sums each
 // particle's records in a fixed order (pairs where it is j, then pairs where
 // it is i, each by pair index), so results do not depend on thread timing.
