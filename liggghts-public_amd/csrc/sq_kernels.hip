@@ -391,13 +391,30 @@ __device__ __forceinline__ bf16x4 get_act(const unsigned short *m, int stride, i
   return v;
 }
 
-// sum over the row of 16 lanes (the tile's samples), by DPP rotations
+template <int CTRL>
+__device__ __forceinline__ float dpp(float v) {
+  return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), CTRL, 0xf, 0xf, true));
+}
+
+// Sums over the row of 16 lanes (the tile's samples), valid in its lane 0: four
+// samples one after another, then the four groups in pairs. The order is part
+// of the result: the parameters after some hundred Adam steps depend on the
+// rounding of each sum.
+constexpr int kDppShl4 = 0x104, kDppShl8 = 0x108;  // the value of lane i + 4, i + 8
+__device__ __forceinline__ float quad_sum(float v) {
+  return ((v + dpp<0x55>(v)) + dpp<0xaa>(v)) + dpp<0xff>(v);  // quad_perm: the quad's lanes 1, 2, 3
+}
+// (group 0 + group 1) + (group 2 + group 3)
 __device__ __forceinline__ float row_sum(float v) {
-  v += __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0x128, 0xf, 0xf, true));
-  v += __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0x124, 0xf, 0xf, true));
-  v += __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0x122, 0xf, 0xf, true));
-  v += __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0x121, 0xf, 0xf, true));
-  return v;
+  v = quad_sum(v);
+  v += dpp<kDppShl4>(v);
+  return v + dpp<kDppShl8>(v);
+}
+// (group 0 + group 2) + (group 1 + group 3)
+__device__ __forceinline__ float row_sum_across(float v) {
+  v = quad_sum(v);
+  v += dpp<kDppShl8>(v);
+  return v + dpp<kDppShl4>(v);
 }
 
 // one gradient pass: every wavefront takes one 16-sample tile of the batch,
@@ -421,12 +438,11 @@ __global__ __launch_bounds__(kBlk) void k_mlp_grad(NetDev net, const float *X, c
   Hidden hid;
   const floatx4 y = forward_tile(net, X, row, valid, hid);
   const float scale = 2.0f / (float)batch;
-  float lsum = 0.f;
-  floatx4 d = {0.f, 0.f, 0.f, 0.f};
+  floatx4 d = {0.f, 0.f, 0.f, 0.f}, sq = d;
   if (valid && q == 0)
     for (int j = 0; j < kOut; j++) {
       const float e = y[j] - T[row * kOut + j];
-      lsum += e * e;
+      sq[j] = e * e;
       d[j] = scale * e;
     }
   const bf16x4 dyb = pack4(d);
@@ -465,7 +481,8 @@ __global__ __launch_bounds__(kBlk) void k_mlp_grad(NetDev net, const float *X, c
     const float b = row_sum(d[j]);
     if (l == 0 && j < kOut) out[kOffB3 + j] = b;
   }
-  lsum = row_sum(lsum);
+  static_assert(kOut == 3, "the loss adds the outputs 0 and 2 first");
+  const float lsum = (row_sum_across(sq[0]) + row_sum_across(sq[2])) + row_sum_across(sq[1]);
   if (l == 0) s.loss[wv] = lsum;
   __syncthreads();  // the tile's operands are in LDS
   // dW3 = H2^T dY, dW2 = H1^T dZ2, dW1 = X^T dZ1 (rows >= kIn are padding)
@@ -505,45 +522,90 @@ __global__ __launch_bounds__(kBlk) void k_mlp_grad(NetDev net, const float *X, c
   }
 }
 
-// sums the blocks' gradient partials (fixed order: deterministic), then one
-// Adam step on the FP32 master parameters and a refresh of the copies the
-// matrix cores read. adam = 0: only the summed gradient is written. 64
-// parameters a block, each summed by 16 threads: one thread a parameter, which
-// leaves 22 blocks with 128 loads in a row each, took 34 us of a step, this
-// takes 5. The last block sums the batch loss.
-constexpr int kAdamParams = 64, kAdamSlices = 16;
-__global__ __launch_bounds__(kAdamParams * kAdamSlices) void k_mlp_adam(NetDev net, const float *part, int nparts,
-                                                                        float *grad, AdamArgs ad) {
-  __shared__ float sum[kAdamSlices][kAdamParams];
+// sums the blocks' gradient partials one after another, then one Adam step on
+// the FP32 master parameters and a refresh of the copies the matrix cores read.
+// ad.apply = 0: only the summed gradient is written. 64 parameters a block: its
+// 1,024 threads load 256 partials of each together, one wavefront adds them in
+// order out of LDS. The last block sums the batch loss. Bound by that chain of
+// additions, about 1 us for the 128 partials of 8,192 samples: a training step
+// takes 25.0 us (16,384 samples: 27.5); with the partials added in 16 slices,
+// another order, 24.1 (25.9), with one thread a parameter loading them in a
+// row 67 (103).
+constexpr int kAdamParams = 64, kAdamSlices = 16, kAdamRows = 256, kAdamBatch = 32;
+__global__ __launch_bounds__(kAdamParams * kAdamSlices)
+    __attribute__((amdgpu_waves_per_eu(4, 4))) void k_mlp_adam(NetDev net, const float *part, int nparts, float *grad,
+                                                               AdamArgs ad) {
+  __shared__ float stage[kAdamRows][kAdamParams];
   const int c = threadIdx.x % kAdamParams, sl = threadIdx.x / kAdamParams;
   const bool loss = blockIdx.x == gridDim.x - 1;
   const int i = blockIdx.x * kAdamParams + c;
-  float v = 0.f;
-  if (loss) {
-    for (int b = threadIdx.x; b < nparts; b += kAdamParams * kAdamSlices) v += ad.loss_part[b];
-  } else if (i < kNumParams) {
-#pragma unroll 8
-    for (int b = sl; b < nparts; b += kAdamSlices) v += part[(int64_t)b * kNumParams + i];
+  const int at = i < kNumParams ? i : kNumParams - 1;
+  // what the update needs is under way while the partials are summed
+  float m0 = 0.f, v0 = 0.f, p0 = 0.f;
+  if (sl == 0 && ad.apply) {
+    m0 = net.m[at];
+    v0 = net.v[at];
+    p0 = net.params[at];
   }
-  sum[sl][c] = v;
-  __syncthreads();
-  if (sl != 0) return;
   float gsum = 0.f;
-  for (int k = 0; k < kAdamSlices; k++) gsum += sum[k][c];
+  for (int b0 = 0; b0 < nparts; b0 += kAdamRows) {
+    const int rows = nparts - b0 < kAdamRows ? nparts - b0 : kAdamRows;
+    const int padded = (rows + kAdamBatch - 1) / kAdamBatch * kAdamBatch;
+    if (b0 > 0) __syncthreads();
+    if (loss) {
+      if ((int)threadIdx.x < padded) stage[threadIdx.x][0] = (int)threadIdx.x < rows ? ad.loss_part[b0 + threadIdx.x] : 0.f;
+    } else {
+      // independent loads, the last row again past it
+      float v[kAdamRows / kAdamSlices];
+#pragma unroll
+      for (int u = 0; u < kAdamRows / kAdamSlices; u++) {
+        const int r = u * kAdamSlices + sl;
+        if (u * kAdamSlices < rows) v[u] = part[(int64_t)(b0 + (r < rows ? r : rows - 1)) * kNumParams + at];
+      }
+#pragma unroll
+      for (int u = 0; u < kAdamRows / kAdamSlices; u++) {
+        const int r = u * kAdamSlices + sl;
+        if (u * kAdamSlices < padded) stage[r][c] = r < rows ? v[u] : 0.f;
+      }
+    }
+    __syncthreads();
+    if (sl == 0) {
+      // the zeros behind the last row change no sum; the next rows are read
+      // while these are added
+      float v[kAdamBatch], w[kAdamBatch];
+      const auto read = [&](float(&q)[kAdamBatch], int r) {
+#pragma unroll
+        for (int u = 0; u < kAdamBatch; u++) q[u] = stage[r + u][c];
+        __builtin_amdgcn_sched_barrier(0);
+      };
+      const auto add = [&](const float(&q)[kAdamBatch]) {
+#pragma unroll
+        for (int u = 0; u < kAdamBatch; u++) gsum += q[u];
+      };
+      read(v, 0);
+      for (int r = 0; r < rows; r += 2 * kAdamBatch) {
+        read(w, r + kAdamBatch < padded ? r + kAdamBatch : 0);
+        add(v);
+        if (r + kAdamBatch >= rows) break;
+        read(v, r + 2 * kAdamBatch < padded ? r + 2 * kAdamBatch : 0);
+        add(w);
+      }
+    }
+  }
+  if (sl != 0) return;
   if (loss) {
-    for (int off = 32; off > 0; off >>= 1) gsum += __shfl_xor(gsum, off, 64);
     if (c == 0 && ad.loss_out) *ad.loss_out = gsum / (float)ad.batch;
     return;
   }
   if (i >= kNumParams) return;
   grad[i] = gsum;
   if (!ad.apply) return;
-  const float m = ad.beta1 * net.m[i] + (1.0f - ad.beta1) * gsum;
-  const float v2 = ad.beta2 * net.v[i] + (1.0f - ad.beta2) * gsum * gsum;
+  const float m = ad.beta1 * m0 + (1.0f - ad.beta1) * gsum;
+  const float v2 = ad.beta2 * v0 + (1.0f - ad.beta2) * gsum * gsum;
   net.m[i] = m;
   net.v[i] = v2;
   const float mh = m / ad.bc1, vh = v2 / ad.bc2;
-  const float p = net.params[i] - ad.lr * mh / (sqrtf(vh) + ad.eps);
+  const float p = p0 - ad.lr * mh / (sqrtf(vh) + ad.eps);
   net.params[i] = p;
   write_packed(net, i, p);
 }
