@@ -505,7 +505,7 @@ template <typename T, bool GEN, typename W>
 __device__ __forceinline__ void mesh_contacts(const StepArgs &a, int i, const double4 &pi,
                                      const double4 &vi, const W &wi, int irow, T &fx, T &fy,
                                      T &fz, T &tx, T &ty, T &tz,
-                                     unsigned long long &nwall) {
+                                     unsigned &nwall) {
   const DevParams &p = a.prm;
   const MeshStep &M = a.mesh;
   const int nc = M.ncand[i];
@@ -1045,7 +1045,7 @@ __device__ __forceinline__ void pair_forces_wave(const StepArgs &a, const Model 
                                                  const int pad, RowWalk walk, const double4 &pi,
                                                  T &fx, T &fy,
                                                  T &fz, T &tx, T &ty, T &tz,
-                                                 unsigned long long &my_contacts,
+                                                 unsigned &my_contacts,
                                                  WaveLds<T, GROUP> &L) {
   typedef typename OmgT<T>::type omg_t;
   const DevParams &p = a.prm;
@@ -1071,7 +1071,7 @@ __device__ __forceinline__ void pair_forces_wave(const StepArgs &a, const Model 
 #pragma unroll
     for (int u = 0; u < GROUP; u++)
       if ((bits >> u) & 1u) L.queue[pos[u]] = make_uint2(ent[u], ((uint32_t)lane << 16) | (uint32_t)ks[u]);
-    my_contacts += (unsigned long long)__popc(bits);
+    my_contacts += (unsigned)__popc(bits);
     wave_sync();
     for (int c0 = 0; c0 < total; c0 += 64) {
       const int q = c0 + lane;
@@ -1154,7 +1154,7 @@ template <typename T, bool GEN, int GROUP>
 __device__ __forceinline__ void pair_forces_rowq(const StepArgs &a, const Model &pm, const int i,
                                                  const int pad, RowWalk walk, T &fx, T &fy,
                                                  T &fz, T &tx, T &ty, T &tz,
-                                                 unsigned long long &my_contacts, RowLds<T> &L) {
+                                                 unsigned &my_contacts, RowLds<T> &L) {
   typedef typename OmgT<T>::type omg_t;
   const DevParams &p = a.prm;
   const size_t cap = (size_t)a.cap;
@@ -1192,7 +1192,7 @@ __device__ __forceinline__ void pair_forces_rowq(const StepArgs &a, const Model 
       }
       if (walk.base == r0) walk.skip();
     }
-    my_contacts += (unsigned long long)c;
+    my_contacts += (unsigned)c;
     int incl = c;
 #pragma unroll
     for (int off = 1; off < 64; off <<= 1) {
@@ -1456,8 +1456,8 @@ __device__ __forceinline__ void finish_particle(const StepArgs &a, const int i, 
 // WAVE 0: each lane resolves its own touching entries.
 template <typename T, bool MESH, int GROUP, bool GEN, int WAVE>
 __device__ __forceinline__ void step_particle(const StepArgs &a, const int i, const bool active,
-                                              unsigned long long &my_contacts,
-                                              unsigned long long &my_wall, int &my_inst,
+                                              unsigned &my_contacts,
+                                              unsigned &my_wall, int &my_inst,
                                               bool &displaced, int &dev, const int reach,
                                               const double *drift, const long long ago_next,
                                               typename PairLdsT<T, GROUP, WAVE>::type *lds) {
@@ -1647,8 +1647,8 @@ __device__ __forceinline__ void group_spread(GroupLds<T> &L, const T f[6],
 // meshes and the integration. 4,000 settled spheres, 500 steps: 12.9 -> 5.8 ms.
 template <typename T, bool MESH, bool GEN, int LANES>
 __device__ __forceinline__ void step_group(const StepArgs &a, const int i,
-                                           unsigned long long &my_contacts,
-                                           unsigned long long &my_wall, int &my_inst,
+                                           unsigned &my_contacts,
+                                           unsigned &my_wall, int &my_inst,
                                            bool &displaced, int &dev, const int reach,
                                            const double *drift, const long long ago_next,
                                            GroupLds<T> &L) {
@@ -1794,6 +1794,10 @@ __device__ __forceinline__ void step_drift(const StepArgs &a, const long long st
     drift[0] = d0[0] + a.prm.dt * v.x;
     drift[1] = d0[1] + a.prm.dt * v.y;
     drift[2] = d0[2] + a.prm.dt * v.z;
+    // the same in every lane: held in scalar registers for the length of the step
+    for (int k = 0; k < 3; k++)
+      drift[k] = __hiloint2double(__builtin_amdgcn_readfirstlane(__double2hiint(drift[k])),
+                                  __builtin_amdgcn_readfirstlane(__double2loint(drift[k])));
   }
 }
 
@@ -1801,10 +1805,10 @@ __device__ __forceinline__ void step_drift(const StepArgs &a, const long long st
 // next step, the contact counts.
 template <int BLOCK>
 __device__ __forceinline__ void step_end(const StepArgs &a, const long long step,
-                                         const unsigned long long my_contacts,
-                                         const unsigned long long my_wall, const bool displaced,
+                                         const unsigned my_contacts,
+                                         const unsigned my_wall, const bool displaced,
                                          const int dev, const int reach) {
-  if (a.prm.reach_on && a.do_initial) raise_reach(a.ctrl, dev, reach);
+  if (reach_counts(a.prm, reach) && a.do_initial) raise_reach(a.ctrl, dev, reach);
   // rebuild request for the next step
   if (__ballot(displaced) != 0ull) {
     if ((threadIdx.x & 63) == 0)
@@ -1844,10 +1848,13 @@ __device__ __forceinline__ void step_end(const StepArgs &a, const long long step
 // meshes into the next step's geometry buffer. Every tile shape computes
 // the same arithmetic in the same order, so results do not depend on it.
 // ---------------------------------------------------------------------------
-// With a mesh the mixed kernel comes to 129 registers, one over what leaves room
-// for four wavefronts per SIMD; asked for four, it takes 128 and spills none.
+// A fourth wavefront per SIMD needs 128 registers or fewer. The mixed Hertz
+// kernels take 120; the sibling models' comes to 134 and, asked for four, takes
+// 128 and spills none (with a mesh it would spill: 135, three wavefronts).
+// Packed beds, mixed, us a step at 144 / 128 registers: epsd2 1M 267 / 251,
+// 400k 113 / 103; hooke + sjkr 1M 203 / 182, 400k 104 / 95.
 template <typename T, bool MESH, int GROUP, bool GEN, int WAVE, int LANES>
-constexpr bool kFourWaves = MESH && sizeof(T) == 4 && GROUP <= 4 && !GEN && WAVE == 0 && LANES == 1;
+constexpr bool kFourWaves = sizeof(T) == 4 && GEN && !MESH && GROUP <= 4 && WAVE == 0 && LANES == 1;
 template <typename T, bool MESH, int BLOCK, int GROUP, bool GEN = false, int WAVE = 0, int LANES = 1>
 __global__ __launch_bounds__(BLOCK)
     __attribute__((amdgpu_waves_per_eu(kFourWaves<T, MESH, GROUP, GEN, WAVE, LANES> ? 4 : 1))) void k_step(StepArgs a) {
@@ -1863,10 +1870,10 @@ __global__ __launch_bounds__(BLOCK)
   constexpr bool kWaveLds = WAVE == 1 || WAVE == 2 || kGrouped;
   __shared__ Lds lds_all[kWaveLds ? BLOCK / 64 : 1];
   Lds *lds = &lds_all[kWaveLds ? (threadIdx.x >> 6) : 0];
-  unsigned long long my_contacts = 0, my_wall = 0;
+  unsigned my_contacts = 0, my_wall = 0;  // of a lane: 32 bits hold them
   bool displaced = false;
   int dev = 0;
-  const int reach = a.ctrl->reach;
+  const int reach = __builtin_amdgcn_readfirstlane(a.ctrl->reach);
   double drift[3];
   step_drift(a, step, drift);
   if (p.reach_on && a.do_initial && blockIdx.x == 0 && threadIdx.x < 3)
@@ -1877,7 +1884,7 @@ __global__ __launch_bounds__(BLOCK)
     const int i = tile * TILE + (int)threadIdx.x / LANES;
     const bool active = i < a.n;
     if ((kWaveLds && !kGrouped) || active) {
-      unsigned long long c = 0, w = 0;
+      unsigned c = 0, w = 0;
       int inst = 0;
       if constexpr (kGrouped)
         step_group<T, MESH, GEN, LANES>(a, i, c, w, inst, displaced, dev, reach, drift, ago_next, *lds);
@@ -1886,8 +1893,8 @@ __global__ __launch_bounds__(BLOCK)
       my_contacts += c;
       my_wall += w;
       if (active && a.count && a.inst_stats) {
-        if (c) atomicAdd(&a.inst_stats[inst], c);
-        if (w) atomicAdd(&a.inst_stats[p.ninst + inst], w);
+        if (c) atomicAdd(&a.inst_stats[inst], (unsigned long long)c);
+        if (w) atomicAdd(&a.inst_stats[p.ninst + inst], (unsigned long long)w);
       }
     }
   }
@@ -1912,10 +1919,10 @@ __global__ __launch_bounds__(kMeshBlock) void k_step_mesh(StepArgs a) {
   const DevParams &p = a.prm;
   long long step, ago_next;
   if (!step_index(a, step, ago_next)) return;
-  unsigned long long my_wall = 0;
+  unsigned my_wall = 0;
   bool displaced = false;
   int dev = 0;
-  const int reach = a.ctrl->reach, listed = a.ctrl->nmesh_near;
+  const int reach = __builtin_amdgcn_readfirstlane(a.ctrl->reach), listed = a.ctrl->nmesh_near;
   double drift[3];
   step_drift(a, step, drift);
   const size_t cap = (size_t)a.cap;
@@ -1935,7 +1942,7 @@ __global__ __launch_bounds__(kMeshBlock) void k_step_mesh(StepArgs a) {
     int meta = meta0;
     T fx = (T)a.fout[i], fy = (T)a.fout[cap + i], fz = (T)a.fout[2 * cap + i];
     T tx = (T)a.fout[3 * cap + i], ty = (T)a.fout[4 * cap + i], tz = (T)a.fout[5 * cap + i];
-    unsigned long long w = 0;
+    unsigned w = 0;
     mesh_contacts<T, GEN>(a, i, pi, vi, wi, irow, fx, fy, fz, tx, ty, tz, w);
     if (p.has_grav && !p.grav_first) {
       fx += (T)(vi.w * p.gacc[0]);
@@ -1945,7 +1952,7 @@ __global__ __launch_bounds__(kMeshBlock) void k_step_mesh(StepArgs a) {
     finish_particle<T>(a, i, pi, vi, wi, fx, fy, fz, tx, ty, tz, meta, displaced, dev, reach, drift, ago_next);
     if (meta != meta0) a.aux.meta[i] = meta;
     my_wall += w;
-    if (a.count && a.inst_stats && w) atomicAdd(&a.inst_stats[p.ninst + inst], w);
+    if (a.count && a.inst_stats && w) atomicAdd(&a.inst_stats[p.ninst + inst], (unsigned long long)w);
   }
   step_end<kMeshBlock>(a, step, 0, my_wall, displaced, dev, reach);
 }
