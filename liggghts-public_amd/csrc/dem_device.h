@@ -267,6 +267,7 @@ struct StepArgs {
   // step's geometry buffer (mv.dst) while the others compute this step
   int variant, pblocks, move_mesh;
   int lanes;           // lanes per particle (1, or 4 or 8 in shape 0)
+  int stretch;         // log2 of the consecutive tiles an XCD walks
   int drift_from;      // k_initial: the drift slot of the last run's final step
   int step_from_ctrl;  // step = ctrl->step_base + step, ago_next = ctrl->ago_base + step
   MeshMoveArgs mv;

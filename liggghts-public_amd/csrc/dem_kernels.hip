@@ -28,21 +28,21 @@ constexpr double kPi = 3.14159265358979323846;  // M_PI
 // ---------------------------------------------------------------------------
 
 // Workgroups are dispatched round-robin over the 8 XCDs (block b -> XCD b%8).
-// Remap so that each XCD walks stretches of kXcdChunk consecutive tiles of
+// Remap so that each XCD walks stretches of 2^stretch consecutive tiles of
 // Morton-ordered particles: the neighbors of a particle then mostly sit in the
-// same XCD's L2 (a stretch's records are under 1 MB of its 4), and the
-// stretches of the XCDs alternate, so that a region with more contacts than
-// the rest (the bottom of a filling) is spread over all of them. One contiguous
-// eighth per XCD left most of the chip waiting for the eighths at the bottom:
-// 700 steps of 1M spheres settling with 270k contacts, mixed 76 -> 59 ms, FP64
-// 108 -> 81 ms; stretches of 4 and 64 tiles measured within 5 % of 16.
-constexpr int kXcdChunk = 16;
-__device__ __forceinline__ int xcd_block(int nblocks) {
+// same XCD's L2, and the stretches of the XCDs alternate, so that a region
+// with more contacts than the rest (the bottom of a filling) is spread over
+// all of them. One contiguous eighth per XCD left most of the chip waiting for
+// the eighths at the bottom: 700 steps of 1M spheres settling with 270k
+// contacts, mixed 76 -> 59 ms, FP64 108 -> 81 ms (16 tiles). The step kernel's
+// stretch is step_stretch's; k_build takes 16 tiles.
+constexpr int kBuildStretch = 4;
+__device__ __forceinline__ int xcd_block(const int nblocks, const int stretch) {
   const int b = blockIdx.x;
-  const int whole = nblocks / (8 * kXcdChunk) * (8 * kXcdChunk);
+  const int whole = nblocks >> (stretch + 3) << (stretch + 3);
   if (b < whole) {
     const int xcd = b & 7, slot = b >> 3;
-    return ((slot / kXcdChunk) * 8 + xcd) * kXcdChunk + slot % kXcdChunk;
+    return ((((slot >> stretch) << 3) + xcd) << stretch) + (slot & ((1 << stretch) - 1));
   }
   // the rest: one stretch per XCD
   const int r = b - whole, n = nblocks - whole;
@@ -1880,7 +1880,7 @@ __global__ __launch_bounds__(BLOCK)
     a.ctrl->drift[(step + 1) & 1][threadIdx.x] = drift[threadIdx.x];
   constexpr int TILE = BLOCK / LANES;
   const int ntiles = (a.n + TILE - 1) / TILE;
-  for (int tile = xcd_block(a.pblocks); tile < ntiles; tile += a.pblocks) {
+  for (int tile = xcd_block(a.pblocks, a.stretch); tile < ntiles; tile += a.pblocks) {
     const int i = tile * TILE + (int)threadIdx.x / LANES;
     const bool active = i < a.n;
     if ((kWaveLds && !kGrouped) || active) {
@@ -2606,7 +2606,7 @@ template <typename T>
 __global__ __launch_bounds__(kBlock) void k_build(RebuildArgs a) {
   __shared__ BuildLds lds;
   const int t = threadIdx.x;
-  const int i = xcd_block(gridDim.x) * kBlock + t;
+  const int i = xcd_block(gridDim.x, kBuildStretch) * kBlock + t;
   const bool active = i < a.n;
   int cnt = 0;
   if (active) {

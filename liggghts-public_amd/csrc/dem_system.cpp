@@ -439,6 +439,9 @@ int step_variant(const dem_handle *h) {
   return ((uses_generic_models(h) || h->hw != 3) && h->variant != 5) ? 0 : h->variant;
 }
 
+// a row holds six entries or more
+bool packed_rows(const dem_handle *h) { return h->npairs >= 3 * h->n; }
+
 // Lanes per particle in the default shape. One lane resolves a particle's
 // contacts one after another (about 20 us for a bed's six), and that chain is
 // the step when there are too few wavefronts to hide it; a group of lanes takes
@@ -452,13 +455,33 @@ int step_variant(const dem_handle *h) {
 //   80,000          30.9 / 31.6 / 39.0   42.8 / 46.2 / 58.4
 // A cloud without contacts has no chain to shorten (4,000: 10.7 / 9.6 / 9.9,
 // 12,000: 9.0 / 8.7 / 9.3, 24,000: 8.6 / 9.2 / 9.9), so the list's length
-// decides as well.
+// decides as well. With a mesh the group's first lane walks the triangles, one
+// lane a particle leaves them to k_step_mesh; the rule holds there too but at
+// its upper end. A run of a drum, mixed, us a step with the rule / one lane:
+// 3,000 spheres 31.8 / 41.1, 8,000 23.4 / 37.1, 16,000 31.5 / 38.6, 24,000
+// 31.9 / 38.7, 36,000 36.7 / 39.0, 48,000 46.7 / 42.5; heaps on a mesh floor,
+// 2,000 16.6 / 25.5, 4,000 17.2 / 29.1, 10,000 18.1 / 29.8.
 int step_lanes(const dem_handle *h) {
   constexpr int64_t kFew = 16 * 1024, kSome = 48 * 1024;
   if (step_variant(h) != 0 || h->persist != 0 || h->n > kSome) return 1;
-  const bool packed = h->npairs >= 3 * h->n;  // a row holds six entries or more
+  const bool packed = packed_rows(h);
   if (h->n <= kFew) return packed ? 8 : 4;
   return packed ? 4 : 1;
+}
+
+// log2 of the consecutive tiles an XCD walks (xcd_block): 16 tiles, or 64 in a
+// large packed bed, whose contacts read their partners' records and so pay for
+// the stretches' borders. With 16, 400k-600k spheres in contact were slower
+// than with one contiguous range per XCD. A step in us, 16 / 64 tiles (one
+// range): compressed packs, mixed, 600k 120 / 115 (115), 400k 91.3 / 89.0
+// (88.9); closed beds of 400k, mixed 76.7 / 73.7 (80.6), FP64 99.4 / 97.3 (107).
+// Below about 1,000 tiles 64 are too coarse a share for 8 XCDs (120k bed mixed
+// 31.5 / 32.6, FP64 with sjkr 41.8 / 43.3; 200k pack mixed 57.4 / 58.6), and a
+// falling cloud, which reads no partner, gains nothing (1M FP64 46.7 / 47.8,
+// 250k mixed 15.0 / 15.5).
+int step_stretch(const dem_handle *h) {
+  constexpr int64_t kMany = 256 * 1024;
+  return packed_rows(h) && h->n >= kMany && step_lanes(h) == 1 ? 6 : 4;
 }
 
 // in_buf: particle state buffer read by the step; tri_buf: geometry buffer of
@@ -487,6 +510,7 @@ dem::StepArgs step_args(dem_handle *h, int in_buf, int tri_buf) {
   a.inst_stats = h->d_inst_stats;
   a.variant = step_variant(h);
   a.lanes = step_lanes(h);
+  a.stretch = step_stretch(h);
   {
     const int B = dem::step_block(a.variant, a.lanes) / a.lanes;
     const int ntiles = (int)((std::max<int64_t>(h->n, 1) + B - 1) / B);
@@ -1745,7 +1769,7 @@ constexpr int kGraphBatch = 32; // steps per captured graph
 // take their step index from the control block (launch_set_base).
 int step_graph(dem_handle *h, int st, int tc, bool moving, hipGraphExec_t *out) {
   const int key = st | (tc << 1) | (h->cur_aux << 2) | (h->variant << 3) | (h->persist << 6) |
-                  ((moving ? 1 : 0) << 13) | (step_lanes(h) << 14);
+                  ((moving ? 1 : 0) << 13) | (step_lanes(h) << 14) | (step_stretch(h) << 18);
   for (auto &g : h->graphs)
     if (g.key == key) {
       *out = g.exec;
