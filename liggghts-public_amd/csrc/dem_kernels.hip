@@ -1361,6 +1361,19 @@ __device__ __forceinline__ int wall_contact(const StepArgs &a, const int i, cons
   return kWallApart;
 }
 
+// The drift the particles' distances are taken from: one particle's path since
+// the build, so that a cloud moving as one keeps its rows' reach. Any common
+// vector serves; it is advanced by that particle's velocity as it stands in
+// this step's input, which every wavefront reads alike. Read where it is used:
+// held from the start of the step it costs the pair phase six registers.
+__device__ __forceinline__ void step_drift(const StepArgs &a, const long long step, double drift[3]) {
+  const double *d0 = a.ctrl->drift[step & 1];
+  const double4 v = a.in.vel[a.n >> 1];
+  drift[0] = d0[0] + a.prm.dt * v.x;
+  drift[1] = d0[1] + a.prm.dt * v.y;
+  drift[2] = d0[2] + a.prm.dt * v.z;
+}
+
 // The end of a particle's step: its force and torque stored when asked for,
 // final integrate of this step, initial integrate of the next.
 template <typename T, typename W>
@@ -1368,7 +1381,7 @@ __device__ __forceinline__ void finish_particle(const StepArgs &a, const int i, 
                                                 const double4 &vi, const W &wi, const T fx,
                                                 const T fy, const T fz, const T tx, const T ty,
                                                 const T tz, int &meta, bool &displaced, int &dev,
-                                                const int reach, const double *drift,
+                                                const int reach, const long long step,
                                                 const long long ago_next) {
   typedef typename OmgT<T>::type omg_t;
   const DevParams &p = a.prm;
@@ -1415,6 +1428,8 @@ __device__ __forceinline__ void finish_particle(const StepArgs &a, const int i, 
       const bool decide = ago_next % p.neigh_every == 0;
       if (p.neigh_check) {
         if (decide || reach_counts(p, reach)) {
+          double drift[3] = {0.0, 0.0, 0.0};
+          if (reach_counts(p, reach)) step_drift(a, step, drift);
           const double hx = x - a.xhold[i];
           const double hy = y - a.xhold[cap + i];
           const double hz = z - a.xhold[2 * cap + i];
@@ -1459,7 +1474,7 @@ __device__ __forceinline__ void step_particle(const StepArgs &a, const int i, co
                                               unsigned &my_contacts,
                                               unsigned &my_wall, int &my_inst,
                                               bool &displaced, int &dev, const int reach,
-                                              const double *drift, const long long ago_next,
+                                              const long long step, const long long ago_next,
                                               typename PairLdsT<T, GROUP, WAVE>::type *lds) {
   typedef typename OmgT<T>::type omg_t;
   const DevParams &p = a.prm;
@@ -1580,7 +1595,7 @@ __device__ __forceinline__ void step_particle(const StepArgs &a, const int i, co
     if (meta != meta0) a.aux.meta[i] = meta;
     return;
   }
-  finish_particle<T>(a, i, pi, vi, wi, fx, fy, fz, tx, ty, tz, meta, displaced, dev, reach, drift, ago_next);
+  finish_particle<T>(a, i, pi, vi, wi, fx, fy, fz, tx, ty, tz, meta, displaced, dev, reach, step, ago_next);
   if (meta != meta0) a.aux.meta[i] = meta;
 }
 
@@ -1650,7 +1665,7 @@ __device__ __forceinline__ void step_group(const StepArgs &a, const int i,
                                            unsigned &my_contacts,
                                            unsigned &my_wall, int &my_inst,
                                            bool &displaced, int &dev, const int reach,
-                                           const double *drift, const long long ago_next,
+                                           const long long step, const long long ago_next,
                                            GroupLds<T> &L) {
   typedef typename OmgT<T>::type omg_t;
   const DevParams &p = a.prm;
@@ -1765,7 +1780,7 @@ __device__ __forceinline__ void step_group(const StepArgs &a, const int i,
   }
   if (sub == 0) {
     finish_particle<T>(a, i, pi, vi, wi, f[0], f[1], f[2], f[3], f[4], f[5], meta, displaced, dev,
-                       reach, drift, ago_next);
+                       reach, step, ago_next);
     if (meta != meta0) a.aux.meta[i] = meta;
   }
 }
@@ -1780,25 +1795,6 @@ __device__ __forceinline__ bool step_index(const StepArgs &a, long long &step, l
     ago_next = a.ctrl->ago_base + a.step;
   }
   return step < a.ctrl->stop_at;
-}
-
-// The drift the particles' distances are taken from: one particle's path since
-// the build, so that a cloud moving as one keeps its rows' reach. Any common
-// vector serves; it is advanced by that particle's velocity as it stands in
-// this step's input, which every wavefront reads alike.
-__device__ __forceinline__ void step_drift(const StepArgs &a, const long long step, double drift[3]) {
-  drift[0] = drift[1] = drift[2] = 0.0;
-  if (a.prm.reach_on && a.do_initial) {
-    const double *d0 = a.ctrl->drift[step & 1];
-    const double4 v = a.in.vel[a.n >> 1];
-    drift[0] = d0[0] + a.prm.dt * v.x;
-    drift[1] = d0[1] + a.prm.dt * v.y;
-    drift[2] = d0[2] + a.prm.dt * v.z;
-    // the same in every lane: held in scalar registers for the length of the step
-    for (int k = 0; k < 3; k++)
-      drift[k] = __hiloint2double(__builtin_amdgcn_readfirstlane(__double2hiint(drift[k])),
-                                  __builtin_amdgcn_readfirstlane(__double2loint(drift[k])));
-  }
 }
 
 // What a block's particles ask for: the reach raised, a rebuild before the
@@ -1849,8 +1845,8 @@ __device__ __forceinline__ void step_end(const StepArgs &a, const long long step
 // the same arithmetic in the same order, so results do not depend on it.
 // ---------------------------------------------------------------------------
 // A fourth wavefront per SIMD needs 128 registers or fewer. The mixed Hertz
-// kernels take 120; the sibling models' comes to 134 and, asked for four, takes
-// 128 and spills none (with a mesh it would spill: 135, three wavefronts).
+// kernels take 120; the sibling models' comes to a few more than 128 and, asked
+// for four, takes 128 and spills none (with a mesh it would: 135, three).
 // Packed beds, mixed, us a step at 144 / 128 registers: epsd2 1M 267 / 251,
 // 400k 113 / 103; hooke + sjkr 1M 203 / 182, 400k 104 / 95.
 template <typename T, bool MESH, int GROUP, bool GEN, int WAVE, int LANES>
@@ -1874,10 +1870,13 @@ __global__ __launch_bounds__(BLOCK)
   bool displaced = false;
   int dev = 0;
   const int reach = __builtin_amdgcn_readfirstlane(a.ctrl->reach);
-  double drift[3];
-  step_drift(a, step, drift);
-  if (p.reach_on && a.do_initial && blockIdx.x == 0 && threadIdx.x < 3)
-    a.ctrl->drift[(step + 1) & 1][threadIdx.x] = drift[threadIdx.x];
+  // (a block that finds the reach past its use sooner than others leaves a
+  // drift that nothing reads before the next build)
+  if (blockIdx.x == 0 && threadIdx.x == 0 && reach_counts(p, reach) && a.do_initial) {
+    double drift[3];
+    step_drift(a, step, drift);
+    for (int k = 0; k < 3; k++) a.ctrl->drift[(step + 1) & 1][k] = drift[k];
+  }
   constexpr int TILE = BLOCK / LANES;
   const int ntiles = (a.n + TILE - 1) / TILE;
   for (int tile = xcd_block(a.pblocks, a.stretch); tile < ntiles; tile += a.pblocks) {
@@ -1887,9 +1886,9 @@ __global__ __launch_bounds__(BLOCK)
       unsigned c = 0, w = 0;
       int inst = 0;
       if constexpr (kGrouped)
-        step_group<T, MESH, GEN, LANES>(a, i, c, w, inst, displaced, dev, reach, drift, ago_next, *lds);
+        step_group<T, MESH, GEN, LANES>(a, i, c, w, inst, displaced, dev, reach, step, ago_next, *lds);
       else
-        step_particle<T, MESH, GROUP, GEN, WAVE>(a, i, active, c, w, inst, displaced, dev, reach, drift, ago_next, lds);
+        step_particle<T, MESH, GROUP, GEN, WAVE>(a, i, active, c, w, inst, displaced, dev, reach, step, ago_next, lds);
       my_contacts += c;
       my_wall += w;
       if (active && a.count && a.inst_stats) {
@@ -1923,8 +1922,6 @@ __global__ __launch_bounds__(kMeshBlock) void k_step_mesh(StepArgs a) {
   bool displaced = false;
   int dev = 0;
   const int reach = __builtin_amdgcn_readfirstlane(a.ctrl->reach), listed = a.ctrl->nmesh_near;
-  double drift[3];
-  step_drift(a, step, drift);
   const size_t cap = (size_t)a.cap;
   // spread over all the blocks, a few lanes of each: there are too few to fill
   // the chip, and a wavefront walks every case its triangles fall into
@@ -1949,7 +1946,7 @@ __global__ __launch_bounds__(kMeshBlock) void k_step_mesh(StepArgs a) {
       fy += (T)(vi.w * p.gacc[1]);
       fz += (T)(vi.w * p.gacc[2]);
     }
-    finish_particle<T>(a, i, pi, vi, wi, fx, fy, fz, tx, ty, tz, meta, displaced, dev, reach, drift, ago_next);
+    finish_particle<T>(a, i, pi, vi, wi, fx, fy, fz, tx, ty, tz, meta, displaced, dev, reach, step, ago_next);
     if (meta != meta0) a.aux.meta[i] = meta;
     my_wall += w;
     if (a.count && a.inst_stats && w) atomicAdd(&a.inst_stats[p.ninst + inst], (unsigned long long)w);
