@@ -167,6 +167,7 @@ struct Ctrl {
   // and the drift it is taken from, of steps of even and odd index
   int reach;
   int nmesh_near;  // particles with candidate triangles at the last build (MeshStep::near)
+  int bad_index;   // k_export met a caller index outside the system
   double drift[2][3];
 };
 
@@ -344,6 +345,7 @@ struct ExportArgs {
 };
 
 // launchers (dem_kernels.hip)
+hipError_t launch_export_begin(const ExportArgs &a, hipStream_t s);  // clears *bad
 hipError_t launch_export(const ExportArgs &a, hipStream_t s);
 hipError_t launch_rebuild(const RebuildArgs &a, hipStream_t s);
 hipError_t launch_step(const StepArgs &a, hipStream_t s);

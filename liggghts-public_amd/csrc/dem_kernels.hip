@@ -3066,9 +3066,13 @@ __global__ __launch_bounds__(kBlock) void k_export(ExportArgs a) {
 // ---------------------------------------------------------------------------
 static inline int nblk(int n, int b) { return (n + b - 1) / b; }
 
+hipError_t launch_export_begin(const ExportArgs &a, hipStream_t s) {
+  hipLaunchKernelGGL(k_zero, dim3(1), dim3(kBlock), 0, s, a.bad, 1);
+  return hipGetLastError();
+}
+
 hipError_t launch_export(const ExportArgs &a, hipStream_t s) {
   if (a.n <= 0) return hipSuccess;
-  hipLaunchKernelGGL(k_zero, dim3(1), dim3(kBlock), 0, s, a.bad, 1);
   if (a.mixed)
     hipLaunchKernelGGL(k_export<float>, dim3(nblk(a.n, kBlock)), dim3(kBlock), 0, s, a);
   else

@@ -126,8 +126,6 @@ struct dem_handle {
   bool setup_done = false;
   bool can_continue = false;  // fout holds the last force pass in the current order
   double *xhold = nullptr, *fout = nullptr;
-  double *export_buf = nullptr;  // dem_get_state: the arrays in caller order, then the flag
-  int64_t export_n = 0;          // particles it has room for, five arrays each
   double rmax = 0.0;
   double rmax_future = 0.0;  // dem_set_max_radius: particles still to come
   // particles waiting to join at the next run's first step (dem_insert_particles)
@@ -237,8 +235,6 @@ void free_particles(dem_handle *h) {
     h->lst[b] = ListBuf{};
   }
   h->xhold = h->fout = nullptr;
-  h->export_buf = nullptr;
-  h->export_n = 0;
   h->d_tri_buf[0] = h->d_tri_buf[1] = nullptr;
   h->d_node_last = nullptr;
   h->d_motion = nullptr;
@@ -2059,17 +2055,13 @@ int dem_get_state(dem_handle *h, double *x, double *v, double *omega, double *f,
   if (h->n <= 0) return DEM_OK;  // an empty system (particles still to be inserted): nothing to copy
   HIPCHK(h, hipSetDevice(h->p.device));
   const int64_t n = h->n;
-  if (n > h->export_n) {
-    HIPCHK(h, hipStreamSynchronize(h->stream));
-    dfree(h, h->export_buf);
-    h->export_buf = nullptr;
-    h->export_n = 0;
-    const int64_t room = std::max<int64_t>(n, h->cap);
-    int rc = dalloc(h, (void **)&h->export_buf, sizeof(double) * (15 * (size_t)room + 1));
-    if (rc) return rc;
-    h->export_n = room;
-  }
-  // reordered on the device, so each array is one contiguous copy
+  // reordered on the device, so each array is one contiguous copy. The state
+  // buffer that the next step or build writes whole holds the reordered arrays
+  // meanwhile, two or three at a time: 24 bytes a particle of its 32, so a
+  // system that fills the card can be read out
+  StateBuf &alt = h->st[1 - h->cur_st];
+  double *room[3] = {(double *)alt.pos, (double *)alt.vel, (double *)alt.omg};
+  const int nroom = h->mixed ? 2 : 3;  // mixed angular velocities are 16 bytes
   dem::ExportArgs e{};
   e.n = (int)n;
   e.cap = h->cap;
@@ -2078,16 +2070,26 @@ int dem_get_state(dem_handle *h, double *x, double *v, double *omega, double *f,
   e.orig = h->aux[h->cur_aux].orig;
   e.fout = h->fout;
   double *dst[5] = {x, v, omega, f, torque};
-  for (int q = 0; q < 5; q++) e.out[q] = dst[q] ? h->export_buf + 3 * (size_t)h->export_n * q : nullptr;
-  e.bad = (int *)(h->export_buf + 15 * (size_t)h->export_n);
-  HIPCHK(h, dem::launch_export(e, h->stream));
-  int bad = 0;
-  HIPCHK(h, hipMemcpyAsync(&bad, e.bad, sizeof(int), hipMemcpyDeviceToHost, h->stream));
-  HIPCHK(h, hipStreamSynchronize(h->stream));
-  if (bad) return fail(h, DEM_ERR_STATE, "corrupt particle index");
-  for (int q = 0; q < 5; q++)
-    if (dst[q])
-      HIPCHK(h, hipMemcpyAsync(dst[q], e.out[q], sizeof(double) * 3 * (size_t)n, hipMemcpyDeviceToHost, h->stream));
+  e.bad = &h->ctrl->bad_index;
+  int &bad = h->ctrl_host->bad_index;
+  HIPCHK(h, dem::launch_export_begin(e, h->stream));
+  for (int q = 0; q < 5;) {
+    int held[3], k = 0;
+    for (int c = 0; c < 5; c++) e.out[c] = nullptr;
+    for (; q < 5 && k < nroom; q++)
+      if (dst[q]) {
+        e.out[q] = room[k];
+        held[k++] = q;
+      }
+    HIPCHK(h, dem::launch_export(e, h->stream));
+    HIPCHK(h, hipMemcpyAsync(&bad, e.bad, sizeof(int), hipMemcpyDeviceToHost, h->stream));
+    // (a copy to pageable memory behind work in flight waits longer than this)
+    HIPCHK(h, hipStreamSynchronize(h->stream));
+    if (bad) return fail(h, DEM_ERR_STATE, "corrupt particle index");
+    for (int c = 0; c < k; c++)
+      HIPCHK(h, hipMemcpyAsync(dst[held[c]], e.out[held[c]], sizeof(double) * 3 * (size_t)n, hipMemcpyDeviceToHost,
+                               h->stream));
+  }
   HIPCHK(h, hipStreamSynchronize(h->stream));
   return DEM_OK;
 }
