@@ -648,7 +648,7 @@ int read_ctrl(dem_handle *h) {
 
 // Neighbor rebuild (verlet.cpp:313-336): FixContactHistory::pre_exchange,
 // Domain::pbc, atom sort, Neighbor::build with history carry-in.
-int rebuild(dem_handle *h) {
+int build_list(dem_handle *h) {
   hipEvent_t e0, e1;
   if (h->timing) {
     HIPCHK(h, hipEventCreate(&e0));
@@ -723,6 +723,13 @@ int rebuild(dem_handle *h) {
   h->npairs = (int64_t)(h->ctrl_host->npairs_full / 2);
   h->nmesh_cand = (int64_t)h->ctrl_host->nmesh_cand;
   return DEM_OK;
+}
+
+int rebuild(dem_handle *h) {
+  const int rc = build_list(h);
+  // the list stays the one of before, but the distances since its build are cleared
+  if (rc) hipMemsetAsync(h->aux[h->cur_aux].lev, 0, sizeof(uint32_t) * (size_t)h->cap, h->stream);
+  return rc;
 }
 
 int force_pass(dem_handle *h, int shearupdate) {
