@@ -226,4 +226,15 @@ __device__ __forceinline__ double pow_tab(const PowTab &t, double x, double y) {
   return ldexp(E2[0] + fma(E2[0], p, E2[1]), k >> 6);
 }
 
+// pow_abs of sq_device.h for x = |x|: 1 for a zero exponent or base 1, 0 for
+// base 0 (to 1e-12); a base that has left every scale stays out of range
+__device__ __forceinline__ double q_pow(const PowTab &t, double x, double y) {
+  const double tol = 1e-12;
+  double r = pow_tab(t, x, y);
+  r = x < 1e300 ? r : (y > 0.0 ? x * x : 1.0 / (x * x));
+  r = x < tol ? 0.0 : r;
+  r = (fabs(y) < tol || fabs(x - 1.0) < tol) ? 1.0 : r;
+  return r;
+}
+
 }  // namespace sqd
