@@ -494,15 +494,18 @@ __global__ __launch_bounds__(kBlk) void k_mlp_grad(NetDev net, const float *X, c
         for (int j = 0; j < 4; j++) out[kOffW3 + (mt * 16 + 4 * q + j) * kOut + r] = g[j];
     }
   }
+  bf16x4 ah[kTilesHid], ax[kTilesIn];
+  for (int mt = 0; mt < kTilesHid; mt++) ah[mt] = get_act(w.h1, kActStride, mt);
+  for (int mt = 0; mt < kTilesIn; mt++) ax[mt] = get_act(w.x, kXStride, mt);
 #pragma unroll
   for (int nt = 0; nt < kTilesHid; nt++) {
     const bf16x4 b2 = get_act(w.d2, kActStride, nt), b1 = get_act(w.d1, kActStride, nt);
     for (int mt = 0; mt < kTilesHid; mt++) {
-      const floatx4 g = mfma(get_act(w.h1, kActStride, mt), b2, zero);
+      const floatx4 g = mfma(ah[mt], b2, zero);
       for (int j = 0; j < 4; j++) out[kOffW2 + (mt * 16 + 4 * q + j) * kHid + nt * 16 + r] = g[j];
     }
     for (int mt = 0; mt < kTilesIn; mt++) {
-      const floatx4 g = mfma(get_act(w.x, kXStride, mt), b1, zero);
+      const floatx4 g = mfma(ax[mt], b1, zero);
       for (int j = 0; j < 4; j++) {
         const int m = mt * 16 + 4 * q + j;
         if (m < kIn) out[kOffW1 + m * kHid + nt * 16 + r] = g[j];
@@ -528,7 +531,7 @@ __global__ __launch_bounds__(kBlk) void k_mlp_grad(NetDev net, const float *X, c
 // 1,024 threads load 256 partials of each together, one wavefront adds them in
 // order out of LDS. The last block sums the batch loss. Bound by that chain of
 // additions, about 1 us for the 128 partials of 8,192 samples: a training step
-// takes 25.0 us (16,384 samples: 27.5); with the partials added in 16 slices,
+// takes 24.7 us (16,384 samples: 27.2); with the partials added in 16 slices,
 // another order, 24.1 (25.9), with one thread a parameter loading them in a
 // row 67 (103).
 constexpr int kAdamParams = 64, kAdamSlices = 16, kAdamRows = 256, kAdamBatch = 32;
