@@ -474,10 +474,12 @@ int step_lanes(const dem_handle *h) {
 // Below about 1,000 tiles 64 are too coarse a share for 8 XCDs (120k bed mixed
 // 31.5 / 32.6, FP64 with sjkr 41.8 / 43.3; 200k pack mixed 57.4 / 58.6), and a
 // falling cloud, which reads no partner, gains nothing (1M FP64 46.7 / 47.8,
-// 250k mixed 15.0 / 15.5).
+// 250k mixed 15.0 / 15.5). Nor does a persistent grid, whose 2,048 blocks at
+// most are four rounds of such stretches (1M pack FP64 in shape 0, 8: 279 /
+// 285, in 7, 8: 262 / 272).
 int step_stretch(const dem_handle *h) {
   constexpr int64_t kMany = 256 * 1024;
-  return packed_rows(h) && h->n >= kMany && step_lanes(h) == 1 ? 6 : 4;
+  return packed_rows(h) && h->n >= kMany && h->persist == 0 ? 6 : 4;
 }
 
 // in_buf: particle state buffer read by the step; tri_buf: geometry buffer of
