@@ -428,6 +428,9 @@ int dem_get_instance_stats(dem_handle *h, int ninst, int64_t *ncontacts, int64_t
  * asks for autotuning: the next runs spend their first batches timing every
  * (variant, persist in {0, 4, 8}) candidate, 8 steps each, in three passes,
  * and keep the fastest. Every shape gives bitwise the same results.
+ * In shape (0, 0), the default, a system of up to 48k particles is stepped by
+ * groups of 4 or 8 lanes per particle in blocks of 64 threads; every other
+ * shape keeps one lane per particle.
  * No reference counterpart (the reference has one CPU loop). */
 int dem_set_step_shape(dem_handle *h, int variant, int persist);
 

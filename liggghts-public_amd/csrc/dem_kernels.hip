@@ -1846,7 +1846,9 @@ __device__ __forceinline__ void step_end(const StepArgs &a, const long long step
 // ---------------------------------------------------------------------------
 // A fourth wavefront per SIMD needs 128 registers or fewer. The mixed Hertz
 // kernels take 120; the sibling models' comes to a few more than 128 and, asked
-// for four, takes 128 and spills none (with a mesh it would: 135, three).
+// for four, takes 128 and spills none (with a mesh it would: 135, three). The
+// frame of 36 B that some of the kernels reserve is not touched by any
+// instruction: scalar registers spilled to lanes of vector ones leave it behind.
 // Packed beds, mixed, us a step at 144 / 128 registers: epsd2 1M 267 / 251,
 // 400k 113 / 103; hooke + sjkr 1M 203 / 182, 400k 104 / 95.
 template <typename T, bool MESH, int GROUP, bool GEN, int WAVE, int LANES>
@@ -1906,12 +1908,13 @@ __global__ __launch_bounds__(BLOCK)
 // They are a few percent of a system and sit in most of its wavefronts, so in
 // k_step every wavefront paid for a triangle search and a contact law that one
 // lane in twenty used, and all of it for their registers (202, two wavefronts
-// per SIMD; 127 and four without). Here they are packed, from the list of the
+// per SIMD; 120 and four without). Here they are packed, from the list of the
 // last build, in no particular order: no particle depends on another. Bound by
 // latency, 15 to 20 us whatever their number. A step in us, the mesh in k_step
 // / here (k_step + k_step_mesh): 727k spheres in 48 heaps on a floor, mixed,
-// 90 / 55 + 15; 250k in a drum, 64 / 44 + 20. In leading blocks of k_step's own
-// launch, whose registers then spill, the two came to 93 and 64.
+// 90 / 54 + 14; 250k in a drum, 64 / 47 + 20: what the drum's step kernel gains
+// the second launch takes again. In leading blocks of k_step's own launch, whose
+// registers then spill, the two came to 93 and 64.
 template <typename T, bool GEN>
 __global__ __launch_bounds__(kMeshBlock) void k_step_mesh(StepArgs a) {
   typedef typename OmgT<T>::type omg_t;

@@ -8,8 +8,8 @@
 // What bounds it: a pair's solve is sequential, and of 100,000 random pairs the
 // slowest takes thousands of iterations, so a launch lasts as long as one
 // pair's chain. One thread per pair took 18 us for each of its iterations:
-// four shape functions (five powers each, issued one after another), a 4 x 4
-// inverse, and 544 B of scratch. Here
+// four shape functions (five powers each, issued one after another) and a 4 x 4
+// inverse, its arrays in scratch memory. Here
 //   - four lanes (a quad) hold one particle: lane c raises local coordinate c
 //     to its power, and lanes 0 and 1 the two powers of x^n2 + y^n2, so a shape
 //     function is two powers deep; the other particle's quad does the same
@@ -19,9 +19,12 @@
 //     without another pair of shape functions;
 //   - lane c owns column c of the Jacobian and forms the four cofactors of
 //     row c of its inverse.
-// Values move inside a row of 16 lanes by DPP (quad_perm, row_ror:8); no LDS.
-// An iteration takes 2.7 us. 100k fresh pairs: 126 -> 21 ms to 228 -> 33 ms by
-// the slowest pair drawn; k_pairs of 50k superquadrics 43 -> 7.4 ms a step.
+// Values move inside a row of 16 lanes by DPP (quad_perm, row_ror:8), not
+// through LDS, which holds the power's tables and what a lane touches rarely.
+// The 880 B of scratch that remain are the GMRES of a nearly singular Jacobian,
+// kept out of line. An iteration takes 2.7 us. 100k fresh pairs: 126 -> 21 ms to
+// 228 -> 33 ms by the slowest pair drawn; the pair kernels of 50k superquadrics
+// (k_pair_start, k_pair_solve, k_pair_finish) 43 -> 7.4 ms a step.
 #pragma once
 
 #include "sq_device.h"

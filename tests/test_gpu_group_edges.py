@@ -1,10 +1,11 @@
 """Sizes at which the work splits of three GPU paths can go wrong.
 
-  contact-point solve   eight lanes per pair, eight pairs per wavefront, the
-                        groups fed from a queue: a pair's result does not depend
-                        on how many pairs there are or where it stands (bitwise),
-                        and equals the oracle's to 1e-12 m (the bound of the
-                        solve's own test) for integer, half and equal blockiness
+  contact-point solve   eight lanes per pair, eight pairs per wavefront, in
+                        batches that give every pair a group of its own: a
+                        pair's result does not depend on how many pairs there
+                        are (bitwise), and 95 % of the points equal the oracle's
+                        to 1e-12 m (the bound of the solve's own test), for
+                        integer, half and equal blockiness
   network gradient      16 samples per tile, tiles spread over the wavefronts:
                         1e-3 norm-wise against the checker with the same BF16
                         rounding points (the bound of the network's own test)
